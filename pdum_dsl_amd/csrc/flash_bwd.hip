@@ -29,6 +29,7 @@
 // body; masked tiles give a masked score its row's pm as probability (0 for
 // any row with a live key) and no gradient (dS = 0), as the where() adjoint.
 #include "attn_common.h"
+#include "attn_f32.h"
 
 #include <type_traits>
 
@@ -785,7 +786,8 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 1) void bwd_main(BwdArgs a) {
 
 // ---------------------------------------------------------------- fp32 column
 //
-// The fp32 backward (any e, od <= 512): the column the reference's f32 runner
+// The fp32 backward for any e, od <= 512 (e = od = 64 or 128 run on the fp32
+// matrix cores, attn_f32.hip): the column the reference's f32 runner
 // occupies for the backward carves (conformance/triton_tile.py). VALU only,
 // one wave per row: bwd_rows_f32<0> owns a query row (dQ), <1> a key row
 // (dK, dV); keys / queries in chunks of 64, one per lane. Row statistics come
@@ -993,13 +995,30 @@ extern "C" int pdh_flash_bwd(const void* q, const void* k, const void* v, const 
     PDH_REQUIRE((ninst * G.t + 3) / 4 <= INT32_MAX && (ninst_kv * G.s + 3) / 4 <= INT32_MAX, PDH_EINVAL,
                 "pdh_flash_bwd: too many rows");
     const int masked = mask_kind == PDH_MASK_BAND;
+    hipStream_t st = as_stream(stream);
+    const int prune_f32 = masked && !band_has_empty_row(G.t, G.s, band_lo, band_hi);
+    if (attn_f32_takes(G) && ninst * G.t * 12 < INT32_MAX) {  // e == od in {64, 128}: the fp32 matrix cores
+      AttnF32Args fa = attn_f32_args(G, scale, fill, masked, band_lo, band_hi, prune_f32);
+      fa.q = static_cast<const float*>(q);
+      fa.k = static_cast<const float*>(k);
+      fa.v = static_cast<const float*>(v);
+      fa.o = const_cast<float*>(static_cast<const float*>(o));
+      fa.dout = static_cast<const float*>(dout);
+      fa.lse = lse;
+      fa.m_in = m_in;
+      fa.den_in = den_in;
+      fa.dq = static_cast<float*>(dq);
+      fa.dk = static_cast<float*>(dk);
+      fa.dv = static_cast<float*>(dv);
+      fa.ws = ws;
+      return attn_f32_backward(fa, G, st);
+    }
     GenBwdArgs ga{static_cast<const float*>(q), static_cast<const float*>(k), static_cast<const float*>(v),
                   static_cast<const float*>(o), static_cast<const float*>(dout), lse, m_in, den_in,
                   static_cast<float*>(dq), static_cast<float*>(dk), static_cast<float*>(dv), ws, ninst * G.t,
                   G.heads_q, G.t, G.s, G.e, G.od, G.heads_kv, group, G.q_sb, G.q_sh, G.q_st, G.k_sb, G.k_sh, G.k_st,
                   G.v_sb, G.v_sh, G.v_st, G.o_sb, G.o_sh, G.o_st, scale, scale * kLog2e, fill * kLog2e, masked,
-                  band_lo, band_hi, masked && !band_has_empty_row(G.t, G.s, band_lo, band_hi)};
-    hipStream_t st = as_stream(stream);
+                  band_lo, band_hi, prune_f32};
     bwd_stats_f32<<<dim3(static_cast<unsigned>((ga.rows + 3) / 4)), 256, 0, st>>>(ga);
     int rc = check_launch("pdh_flash_bwd (fp32 row stats)");
     if (rc) return rc;

@@ -36,10 +36,13 @@
 //     groups of four of alternating direction, so each of an XCD's four
 //     shader engines receives the same total work.
 //
-// Generic fp32 kernel (any e, od, t, s): one wave per query row, keys in
-// chunks of 64 (one per lane), the same recurrence in fp32 — the column the
-// reference's f32 Triton runner occupies (conformance/triton_tile.py:662-698).
+// fp32, the column the reference's f32 Triton runner occupies
+// (conformance/triton_tile.py:662-698): e = od = 64 or 128 run on the fp32
+// matrix cores (attn_f32.hip), e = od = 32 on the row kernel below, any other
+// e, od on the generic kernel (one wave per query row, keys in chunks of 64,
+// one per lane, the same recurrence).
 #include "attn_common.h"
+#include "attn_f32.h"
 
 #include <type_traits>
 
@@ -605,7 +608,7 @@ __global__ __launch_bounds__(256) void flash_fwd_generic_f32(GenArgs a, int64_t 
   }
 }
 
-// The fp32 kernel for heads of E = OD = 32 or 64 features: lane = query
+// The fp32 kernel for heads of E = OD = 32 features: lane = query
 // row, 64 rows per workgroup, so each lane runs its own row's recurrence with
 // no cross-lane reduction, and a key's K and V rows are the same for every
 // lane. The workgroup copies each 64-key chunk of K and V (coalesced rows,
@@ -904,23 +907,30 @@ int flash_fwd_impl(const void* q, const void* k, const void* v, void* o, float* 
   if (dtype == PDH_F32) {
     PDH_REQUIRE(G.od <= 64 * kGenOdPerLane, PDH_EUNSUPPORTED, "pdh_flash_fwd: fp32 od > %d not supported",
                 64 * kGenOdPerLane);
+    if (attn_f32_takes(G)) {  // e == od in {64, 128}: the fp32 matrix cores
+      AttnF32Args fa = attn_f32_args(G, scale, fill, masked, band_lo, band_hi, prune_ok);
+      fa.q = static_cast<const float*>(q);
+      fa.k = static_cast<const float*>(k);
+      fa.v = static_cast<const float*>(v);
+      fa.o = static_cast<float*>(o);
+      fa.m_out = m_out;
+      fa.den_out = den_out;
+      fa.lse_out = lse_out;
+      return attn_f32_forward(fa, G, st);
+    }
     GenArgs ga{static_cast<const float*>(q), static_cast<const float*>(k), static_cast<const float*>(v),
                static_cast<float*>(o), m_out, den_out, lse_out, G.heads_q, G.heads_kv, G.t, G.s, G.e, G.od,
                G.q_sb, G.q_sh, G.q_st, G.k_sb, G.k_sh, G.k_st, G.v_sb, G.v_sh, G.v_st, G.o_sb, G.o_sh, G.o_st,
                scale, fill, masked, band_lo, band_hi, prune_ok};
     const int64_t nrows = ninst * G.t;
-    if (G.e == G.od && (G.e == 32 || G.e == 64)) {  // lanes are rows, K / V rows uniform
+    if (G.e == G.od && G.e == 32) {  // lanes are rows, K / V rows uniform
       const int64_t nqb = (G.t + 63) / 64;
       PDH_REQUIRE(ninst * nqb <= INT32_MAX && nqb <= INT32_MAX, PDH_EINVAL, "pdh_flash_fwd: too many rows");
       const dim3 grid(static_cast<unsigned>(ninst * nqb));
       static int cus = 0;  // compute units, read once (one device per process)
       if (cus == 0) cus = pdh_device_cus() > 0 ? pdh_device_cus() : 256;
       const bool small = ninst * nqb < cus;  // under one workgroup per compute unit
-      if (G.e == 64 && small)
-        flash_fwd_rows_f32_lds<64, 64, 8><<<grid, 512, 0, st>>>(ga, static_cast<int>(nqb));
-      else if (G.e == 64)
-        flash_fwd_rows_f32_lds<64, 64, 4><<<grid, 256, 0, st>>>(ga, static_cast<int>(nqb));
-      else if (small)
+      if (small)
         flash_fwd_rows_f32_lds<32, 32, 8><<<grid, 512, 0, st>>>(ga, static_cast<int>(nqb));
       else
         flash_fwd_rows_f32_lds<32, 32, 4><<<grid, 256, 0, st>>>(ga, static_cast<int>(nqb));
