@@ -192,4 +192,6 @@ def check(fn: str, code: int) -> None:
 
 def call(fn: str, *args) -> None:
     """Call a status-returning entry point; raise PdhError on failure."""
-    check(fn, getattr(lib(), fn)(*args))
+    code = getattr(_lib or lib(), fn)(*args)
+    if code != PDH_OK:
+        check(fn, code)

@@ -39,6 +39,53 @@ struct Entry {
 std::mutex g_mu;
 std::unordered_map<std::string, Entry> g_cache;
 
+// The entry of each request under a short key of exactly what the generated
+// source depends on, so that a launch does not generate the source again to
+// look it up (6 us a call). A source has few keys, and entries stay put in
+// the map above. Guarded by g_mu.
+std::unordered_map<std::string, const Entry*> g_by_request;
+
+template <typename T>
+void key_add(std::string& k, const T& v) {
+  k.append(reinterpret_cast<const char*>(&v), sizeof(T));
+}
+
+// What gen_eval reads of a program: its instructions, and which views are
+// contiguous along the last dim.
+void key_program(std::string& k, const pdh_ew_program& p) {
+  key_add(k, p.n_insns);
+  key_add(k, p.ndim);
+  key_add(k, p.out_reg);
+  uint32_t contiguous = p.out_stride[p.ndim - 1] == 1 ? 1u : 0u;
+  for (int i = 0; i < PDH_EW_MAX_OPERANDS; ++i) contiguous |= p.in_stride[i][p.ndim - 1] == 1 ? 2u << i : 0u;
+  key_add(k, contiguous);
+  for (int i = 0; i < p.n_insns; ++i) {
+    const pdh_ew_insn& in = p.insns[i];
+    const uint8_t b[5] = {in.op, in.dst, in.a, in.b, in.c};
+    key_add(k, b);
+    key_add(k, in.imm);
+  }
+}
+
+std::string request_key(char what, int dev, int dt, int lay, int red) {
+  std::string k;
+  k.reserve(256);
+  k.push_back(what);
+  for (const int v : {dev, dt, lay, red, f32_contract_mode()}) key_add(k, v);
+  return k;
+}
+
+// The entry of request `key` into fns; false when there is none (or the interpreter runs it). known: whether there is one.
+bool find_request(const std::string& key, hipFunction_t fns[2], bool* known) {
+  std::lock_guard<std::mutex> lock(g_mu);
+  const auto it = g_by_request.find(key);
+  *known = it != g_by_request.end();
+  if (!*known || !it->second->ok) return false;
+  fns[0] = it->second->fn[0];
+  fns[1] = it->second->fn[1];
+  return true;
+}
+
 const char* dt_name(int dt) { return dt == PDH_F32 ? "PDH_F32" : dt == PDH_BF16 ? "PDH_BF16" : "PDH_F16"; }
 
 std::string fmt_float(float v) {
@@ -289,21 +336,17 @@ bool jit_enabled() {
   return m == 1;
 }
 
-// The specialized kernel(s) for program p: fn[0] and fn[1] (the one-element
-// map-chain variant; the 64 x 64-tile contraction), or false when the
-// interpreter must run it.
-bool jit_get(JitKind kind, const pdh_ew_program& p, int dt, hipFunction_t fns[2], int lay, int red) {
-  if (!jit_enabled()) return false;
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess) return false;
-  const std::string src = full_source(kind, p, dt, lay, red);
-  const std::string key = std::to_string(dev) + "|" + src;
+namespace {
+
+// The entry of `src` (compiled on its first request) into fns, kept under `key` for the next one.
+bool get(const std::string& key, int dev, const std::string& src, bool two, hipFunction_t fns[2]) {
+  const std::string skey = std::to_string(dev) + "|" + src;
   std::lock_guard<std::mutex> lock(g_mu);
-  auto it = g_cache.find(key);
+  auto it = g_cache.find(skey);
   if (it == g_cache.end()) {
     Entry e;
     std::string err;
-    e.ok = compile(src, kind == JitKind::MapChain || dt != PDH_F32 || f32_contract_mode() != 0, &e, &err);
+    e.ok = compile(src, two, &e, &err);
     if (e.ok)
       ++g_compiled;
     else {
@@ -311,12 +354,31 @@ bool jit_get(JitKind kind, const pdh_ew_program& p, int dt, hipFunction_t fns[2]
       std::fprintf(stderr, "libpdhip: runtime specialization unavailable, the interpreter runs this program (%s)\n",
                    err.c_str());
     }
-    it = g_cache.emplace(key, e).first;
+    it = g_cache.emplace(skey, e).first;
   }
+  g_by_request.emplace(key, &it->second);
   if (!it->second.ok) return false;
   fns[0] = it->second.fn[0];
   fns[1] = it->second.fn[1];
   return true;
+}
+
+}  // namespace
+
+// The specialized kernel(s) for program p: fn[0] and fn[1] (the one-element
+// map-chain variant; the 64 x 64-tile contraction), or false when the
+// interpreter must run it.
+bool jit_get(JitKind kind, const pdh_ew_program& p, int dt, hipFunction_t fns[2], int lay, int red) {
+  if (!jit_enabled()) return false;
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return false;
+  std::string key = request_key(kind == JitKind::MapChain ? 'm' : 'c', dev, dt, lay, red);
+  key_program(key, p);
+  bool known;
+  const bool found = find_request(key, fns, &known);
+  return known ? found
+               : get(key, dev, full_source(kind, p, dt, lay, red),
+                     kind == JitKind::MapChain || dt != PDH_F32 || f32_contract_mode() != 0, fns);
 }
 
 // The specialized row-reduce kernels for (summand, epilogue): fns[0] one
@@ -325,27 +387,12 @@ bool jit_get_reduce(const pdh_ew_program& ps, const pdh_ew_program& pe, int dt, 
   if (!jit_enabled()) return false;
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess) return false;
-  const std::string src = reduce_source(ps, pe, dt);
-  const std::string key = std::to_string(dev) + "|" + src;
-  std::lock_guard<std::mutex> lock(g_mu);
-  auto it = g_cache.find(key);
-  if (it == g_cache.end()) {
-    Entry e;
-    std::string err;
-    e.ok = compile(src, true, &e, &err);
-    if (e.ok)
-      ++g_compiled;
-    else {
-      ++g_failed;
-      std::fprintf(stderr, "libpdhip: runtime specialization unavailable, the interpreter runs this program (%s)\n",
-                   err.c_str());
-    }
-    it = g_cache.emplace(key, e).first;
-  }
-  if (!it->second.ok) return false;
-  fns[0] = it->second.fn[0];
-  fns[1] = it->second.fn[1];
-  return true;
+  std::string key = request_key('r', dev, dt, 0, 0);
+  key_program(key, ps);
+  key_program(key, pe);
+  bool known;
+  const bool found = find_request(key, fns, &known);
+  return known ? found : get(key, dev, reduce_source(ps, pe, dt), true, fns);
 }
 
 // The fp32 prologue kernels specialized for (epilogue, prologues): fns[0] the
@@ -356,27 +403,13 @@ bool jit_get_pro(const pdh_ew_program& pe, const pdh_ew_program* pa, const pdh_e
   if (!jit_enabled()) return false;
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess) return false;
-  const std::string src = pro_source(pe, pa, pb, lay, dt);
-  const std::string key = std::to_string(dev) + "|" + src;
-  std::lock_guard<std::mutex> lock(g_mu);
-  auto it = g_cache.find(key);
-  if (it == g_cache.end()) {
-    Entry e;
-    std::string err;
-    e.ok = compile(src, dt != PDH_F32 || f32_contract_mode() != 0, &e, &err);
-    if (e.ok)
-      ++g_compiled;
-    else {
-      ++g_failed;
-      std::fprintf(stderr, "libpdhip: runtime specialization unavailable, the interpreter runs this program (%s)\n",
-                   err.c_str());
-    }
-    it = g_cache.emplace(key, e).first;
-  }
-  if (!it->second.ok) return false;
-  fns[0] = it->second.fn[0];
-  fns[1] = it->second.fn[1];
-  return true;
+  std::string key = request_key('p', dev, dt, lay, (pa != nullptr ? 1 : 0) | (pb != nullptr ? 2 : 0));
+  key_program(key, pe);
+  if (pa != nullptr) key_program(key, *pa);
+  if (pb != nullptr) key_program(key, *pb);
+  bool known;
+  const bool found = find_request(key, fns, &known);
+  return known ? found : get(key, dev, pro_source(pe, pa, pb, lay, dt), dt != PDH_F32 || f32_contract_mode() != 0, fns);
 }
 
 void jit_count_launch() { ++g_launched; }

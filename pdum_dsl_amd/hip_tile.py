@@ -281,7 +281,8 @@ def recognize_layernorm(region: Region):
 def _torch():
     import torch
 
-    if not torch.cuda.is_available():
+    # an initialized context is a visible GPU (is_available asks the driver each time)
+    if not torch.cuda.is_initialized() and not torch.cuda.is_available():
         raise RuntimeError("compile_tile_hip runners launch HIP kernels: no GPU is visible")
     return torch
 
@@ -345,8 +346,18 @@ def _finish(dev, source: str, grid: int, template: str, region: Region, dtype: s
         for t, shp in zip(tensors, shapes):
             if tuple(t.shape) != shp:
                 raise ValueError(f"a param tensor has shape {tuple(t.shape)}, the region wants {shp}")
-        with torch.cuda.stream(stream) if stream is not None else contextlib.nullcontext():
-            return dev([t.to(device="cuda", dtype=tdt).contiguous() for t in tensors])
+        if stream is not None:
+            with torch.cuda.stream(stream):
+                return dev(placed(torch, tensors, tdt))
+        return dev(placed(torch, tensors, tdt))
+
+    def placed(torch, tensors, tdt):
+        """Dense tensors of the column's type on the current device (as they are, where they already are that)."""
+        if not torch.cuda.is_initialized():
+            torch.cuda.init()
+        here = torch.cuda.current_device()
+        return [t if t.is_cuda and t.dtype is tdt and t.get_device() == here and t.is_contiguous()
+                else t.to(device="cuda", dtype=tdt).contiguous() for t in tensors]
 
     def run(values):
         torch = _torch()
@@ -513,6 +524,15 @@ def _arrange(torch, t, names, order, pad_last=None):
     return x
 
 
+def _dense(shape) -> list:
+    """Element strides of a dense tensor."""
+    st, acc = [], 1
+    for n in reversed(shape):
+        st.insert(0, acc)
+        acc *= n
+    return st
+
+
 def _map_chain_runner(region, grid, dtype):
     from . import ewprog
     from . import kernels as K
@@ -528,18 +548,28 @@ def _map_chain_runner(region, grid, dtype):
     out_names = y.type.names
     shifted = low.offset_reads()
 
+    shape = tuple(d.size for d in dims)
+    bound: list = []  # (program, element offsets), made by the first call: every param is dense, so neither changes
+
     def dev(ts):
         torch = _torch()
-        ops, strides = [], []
+        tdt = getattr(torch, _TORCH_DT[dtype])
+        out = torch.empty(shape, device="cuda", dtype=tdt)
+        if bound:
+            prog, offs = bound[0]
+            return K.map_chain_bound(prog, [ts[i].data_ptr() + o for i, o in zip(idx, offs)], out)
+        ops, strides, offs = [], [], []
         for j, (i, base) in enumerate(zip(idx, low.bases)):
             t = ts[i]  # each param once; shifted reads are offset views of it
-            st, off = low.operand_view(j, dict(zip(base.type.names, t.stride())))
+            st, off = low.operand_view(j, dict(zip(base.type.names, _dense(t.shape))))
             if off < 0:
                 raise Untranslatable("a shifted read starts before its tensor")
             ops.append(t.reshape(-1)[off:])
             strides.append(st)
-        out = torch.empty(tuple(d.size for d in dims), device="cuda", dtype=getattr(torch, _TORCH_DT[dtype]))
-        K.map_chain(low.program(out.stride(), strides), ops, out)
+            offs.append(off * t.element_size())
+        prog = low.program(_dense(shape), strides)
+        K.map_chain(prog, ops, out)  # checks every view against its operand's extent
+        bound.append((prog, offs))
         return out
 
     tmpl = "stencil" if shifted else "map-chain"
@@ -701,6 +731,12 @@ def _contraction_runner(region, cb, grid, dtype):
     epi_idx = [_index(region, p) for p in epi.bases]
 
     fused = dtype in ("f32", "bf16") and "chain" in (pa[0], pb[0])
+    bound: list = []  # the epilogue program
+    present = [nm for nm in lnames if nm in y.type.names]  # the unit stand-ins drop out
+    full_shape = tuple(size[nm].size for nm in present)
+    full_perm = [present.index(nm) for nm in y.type.names]
+    if full_perm == list(range(len(present))):
+        full_perm = None
 
     def dev(ts):
         torch = _torch()
@@ -724,7 +760,10 @@ def _contraction_runner(region, cb, grid, dtype):
             return buf
 
         ops = [ts[i] for i in epi_idx]
-        st = [ewprog.strides_over(t.stride(), p.type.names, lattice) for t, p in zip(ops, epi.operands)]
+        if not bound:  # every param and the output are dense: the program is made by the first call
+            st = [ewprog.strides_over(_dense(t.shape), p.type.names, lattice) for t, p in zip(ops, epi.operands)]
+            bound.append(epi.program(_dense((B_, M_, N_)), st))
+        prog = bound[0]
         out = torch.empty((B_, M_, N_), device="cuda", dtype=tdt)
         if fused:  # chain operands evaluated in the k loop, params read as packed
             sides = []
@@ -738,15 +777,13 @@ def _contraction_runner(region, cb, grid, dtype):
                     t = build(spec, node, order, rows)
                     sides.append((t, t.stride(), None))
             (a, sta, pra), (bt, stb, prb) = sides
-            K.contract_views_pro(a, sta, bt, stb, (B_, M_, N_, Kdim), epi.program(out.stride(), st), ops, out,
-                                 pro_a=pra, pro_b=prb)
+            K.contract_views_pro(a, sta, bt, stb, (B_, M_, N_, Kdim), prog, ops, out, pro_a=pra, pro_b=prb)
         else:
             a = build(pa, cb["a"], a_order, M_)
             bt = build(pb, cb["b"], b_order, N_)
-            K.contract(a, bt, Kdim, epi.program(out.stride(), st), ops, out)
-        present = [nm for nm in lnames if nm in y.type.names]  # the unit stand-ins drop out
-        full = out.reshape(tuple(size[nm].size for nm in present))
-        return full.permute([present.index(nm) for nm in y.type.names])
+            K.contract(a, bt, Kdim, prog, ops, out)
+        full = out.view(full_shape)
+        return full if full_perm is None else full.permute(full_perm)
 
     kern = "contract_views_pro" if fused else ("contract_f32" if dtype == "f32" else f"contract_mfma<{dtype}>")
     src = (f"hip:{kern} batch={B_} m={M_} n={N_} k={Kdim} kp={KP} prologue={pa[0]},{pb[0]} "

@@ -31,11 +31,26 @@ _DT = {torch.float32: PDH_F32, torch.bfloat16: PDH_BF16, torch.float16: PDH_F16}
 
 
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    """The current device's current stream, without the wrapper objects of
+    torch.cuda.current_stream() (2.9 us a call against 0.1)."""
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def _ptr(t: torch.Tensor | None):
-    return None if t is None else C.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
+
+
+_CUS: dict = {}  # device -> compute units
+
+
+def _cus() -> int:
+    if not torch.cuda.is_initialized():
+        return _lib.lib().pdh_device_cus() or 256
+    dev = torch._C._cuda_getDevice()
+    n = _CUS.get(dev)
+    if n is None:
+        n = _CUS[dev] = _lib.lib().pdh_device_cus() or 256
+    return n
 
 
 def _require_cuda(*ts: torch.Tensor) -> None:
@@ -65,30 +80,36 @@ CAUSAL = Band(None, 0)
 # ---------------------------------------------------------------------- rows
 
 
+def _rows(x: torch.Tensor) -> torch.Tensor:
+    """x as [rows, cols] with contiguous columns (a copy where its layout has none)."""
+    if x.dim() == 2 and x.shape[1] > 0 and x.stride(1) == 1:
+        return x
+    x2 = x.reshape(-1, x.shape[-1])
+    return x2 if x2.stride(-1) == 1 else x2.contiguous()
+
+
 def row_softmax(x: torch.Tensor, out: torch.Tensor | None = None) -> torch.Tensor:
     """softmax over the last axis (rows = all leading dims); fp32, bf16 or
     f16 storage, fp32 arithmetic."""
     _require_cuda(x)
     if x.dtype not in _DT:
         raise ValueError(f"row_softmax stores f32, bf16 or f16 (got {x.dtype})")
-    x2 = x.reshape(-1, x.shape[-1])
-    if x2.stride(-1) != 1:
-        x2 = x2.contiguous()
+    x2 = _rows(x)
     y = torch.empty_like(x2) if out is None else out.reshape(-1, x.shape[-1])
     if y.dtype != x.dtype or y.stride(-1) != 1:
         raise ValueError("out must share x's element type and have contiguous rows")
     if x.dtype == torch.float32:
         _lib.call(
             "pdh_row_softmax",
-            _ptr(x2), _ptr(y), x2.shape[0], x2.shape[1], x2.stride(0), y.stride(0), C.c_void_p(_stream()),
+            _ptr(x2), _ptr(y), x2.shape[0], x2.shape[1], x2.stride(0), y.stride(0), _stream(),
         )
     else:
         _lib.call(
             "pdh_row_softmax_dt",
             _ptr(x2), _ptr(y), x2.shape[0], x2.shape[1], x2.stride(0), y.stride(0), _DT[x.dtype],
-            C.c_void_p(_stream()),
+            _stream(),
         )
-    return y.reshape(x.shape)
+    return y if y.shape == x.shape else y.reshape(x.shape)
 
 
 def layernorm(
@@ -110,9 +131,7 @@ def layernorm(
     for nm, t in (("gamma", gamma), ("beta", beta)):
         if t is not None and (t.numel() != n or not t.is_contiguous()):
             raise ValueError(f"{nm} must be a contiguous vector of {n} elements")
-    x2 = x.reshape(-1, n)
-    if x2.stride(-1) != 1:
-        x2 = x2.contiguous()
+    x2 = _rows(x)
     y = torch.empty_like(x2) if out is None else out.reshape(-1, n)
     if y.dtype != x.dtype or y.stride(-1) != 1:
         raise ValueError("out must share x's element type and have contiguous rows")
@@ -120,15 +139,15 @@ def layernorm(
         _lib.call(
             "pdh_layernorm",
             _ptr(x2), _ptr(gamma), _ptr(beta), _ptr(y), x2.shape[0], n, x2.stride(0), y.stride(0),
-            C.c_float(eps), C.c_void_p(_stream()),
+            float(eps), _stream(),
         )
     else:
         _lib.call(
             "pdh_layernorm_dt",
             _ptr(x2), _ptr(gamma), _ptr(beta), _ptr(y), x2.shape[0], n, x2.stride(0), y.stride(0),
-            C.c_float(eps), _DT[x.dtype], C.c_void_p(_stream()),
+            float(eps), _DT[x.dtype], _stream(),
         )
-    return y.reshape(x.shape)
+    return y if y.shape == x.shape else y.reshape(x.shape)
 
 
 def take_rows(table: torch.Tensor, idx: torch.Tensor, out: torch.Tensor | None = None,
@@ -153,7 +172,7 @@ def take_rows(table: torch.Tensor, idx: torch.Tensor, out: torch.Tensor | None =
     _lib.call(
         "pdh_take_rows",
         _ptr(rows), _ptr(flat), _ptr(y), flat.numel(), rows.shape[1], rows.shape[0], rows.stride(0), y.stride(0),
-        _DT[table.dtype], _ptr(bad), C.c_void_p(_stream()),
+        _DT[table.dtype], _ptr(bad), _stream(),
     )
     return y.reshape(tuple(idx.shape) + tuple(table.shape[1:]))
 
@@ -192,7 +211,7 @@ def scatter_add_rows(values: torch.Tensor, idx: torch.Tensor, n_rows: int, out: 
     _lib.call(
         "pdh_scatter_add_rows",
         _ptr(rows), _ptr(flat), _ptr(y), n, rows.shape[1], n_rows, max(rows.stride(0), rows.shape[1]), y.stride(0),
-        _DT[values.dtype], _ptr(bad), C.c_void_p(_stream()),
+        _DT[values.dtype], _ptr(bad), _stream(),
     )
     return y.reshape((n_rows,) + rest)
 
@@ -201,26 +220,20 @@ def scatter_add_rows(values: torch.Tensor, idx: torch.Tensor, n_rows: int, out: 
 
 
 def _geom(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, o: torch.Tensor) -> AttnGeom:
-    for nm, t in (("q", q), ("k", k), ("v", v), ("o", o)):
-        if t.dim() != 4:
+    sq, sk, sv, so = q.stride(), k.stride(), v.stride(), o.stride()
+    for nm, t, st in (("q", q, sq), ("k", k, sk), ("v", v, sv), ("o", o, so)):
+        if len(st) != 4:
             raise ValueError(f"{nm} must be [batch, heads, rows, features] (got shape {tuple(t.shape)})")
-        if t.stride(-1) != 1:
+        if st[3] != 1:
             raise ValueError(f"{nm}'s feature axis must be contiguous")
-    B, Hq, T, E = q.shape
-    Bk, Hkv, S, Ek = k.shape
-    if (Bk, Ek) != (B, E) or v.shape[:3] != k.shape[:3] or o.shape[:3] != q.shape[:3] or o.shape[3] != v.shape[3]:
-        raise ValueError(
-            f"shape mismatch: q {tuple(q.shape)} k {tuple(k.shape)} v {tuple(v.shape)} o {tuple(o.shape)}"
-        )
+    nq, nk, nv, no = tuple(q.shape), tuple(k.shape), tuple(v.shape), tuple(o.shape)
+    B, Hq, T, E = nq
+    Bk, Hkv, S, Ek = nk
+    if Bk != B or Ek != E or nv[:3] != nk[:3] or no[:3] != nq[:3] or no[3] != nv[3]:
+        raise ValueError(f"shape mismatch: q {nq} k {nk} v {nv} o {no}")
     if Hq % Hkv:
         raise ValueError(f"query heads ({Hq}) must be a multiple of key/value heads ({Hkv})")
-    g = AttnGeom()
-    g.batch, g.heads_q, g.heads_kv, g.t, g.s, g.e, g.od = B, Hq, Hkv, T, S, E, v.shape[3]
-    g.q_sb, g.q_sh, g.q_st = q.stride(0), q.stride(1), q.stride(2)
-    g.k_sb, g.k_sh, g.k_st = k.stride(0), k.stride(1), k.stride(2)
-    g.v_sb, g.v_sh, g.v_st = v.stride(0), v.stride(1), v.stride(2)
-    g.o_sb, g.o_sh, g.o_st = o.stride(0), o.stride(1), o.stride(2)
-    return g
+    return AttnGeom(B, Hq, Hkv, T, S, E, nv[3], *sq[:3], *sk[:3], *sv[:3], *so[:3])
 
 
 @dataclass
@@ -256,12 +269,11 @@ def flash_fwd(
     if not (q.dtype == k.dtype == v.dtype) or q.dtype not in _DT:
         raise ValueError(f"q/k/v must share one dtype of f32/bf16/f16 (got {q.dtype}, {k.dtype}, {v.dtype})")
     B, H, T, _ = q.shape
-    o = torch.empty(q.shape[:3] + (v.shape[3],), dtype=q.dtype, device=q.device) if out is None else out
+    o = q.new_empty((B, H, T, v.shape[3])) if out is None else out
     g = _geom(q, k, v, o)
-    st = dict(dtype=torch.float32, device=q.device)
-    lse = torch.empty((B, H, T), **st) if want_lse else None
-    m = torch.empty((B, H, T), **st) if want_artifacts else None
-    den = torch.empty((B, H, T), **st) if want_artifacts else None
+    lse = q.new_empty((B, H, T), dtype=torch.float32) if want_lse else None
+    m = q.new_empty((B, H, T), dtype=torch.float32) if want_artifacts else None
+    den = q.new_empty((B, H, T), dtype=torch.float32) if want_artifacts else None
     sc = 1.0 / math.sqrt(q.shape[3]) if scale is None else float(scale)
     kind, (lo, hi) = (PDH_MASK_NONE, (0, 0)) if band is None else (PDH_MASK_BAND, band.c_args())
     if nsplit is None:
@@ -272,14 +284,14 @@ def flash_fwd(
         _lib.call(
             "pdh_flash_fwd_split",
             _ptr(q), _ptr(k), _ptr(v), _ptr(o), _ptr(m), _ptr(den), _ptr(lse), C.byref(g), _DT[q.dtype],
-            C.c_float(sc), C.c_float(fill), kind, lo, hi, int(bool(prune)), int(nsplit), _ptr(ws),
-            C.c_size_t(ws.numel() * 4), C.c_void_p(_stream()),
+            sc, float(fill), kind, lo, hi, int(bool(prune)), int(nsplit), _ptr(ws),
+            ws.numel() * 4, _stream(),
         )
         return FlashOut(o, lse, m, den)
     _lib.call(
         "pdh_flash_fwd",
         _ptr(q), _ptr(k), _ptr(v), _ptr(o), _ptr(m), _ptr(den), _ptr(lse), C.byref(g), _DT[q.dtype],
-        C.c_float(sc), C.c_float(fill), kind, lo, hi, int(bool(prune)), C.c_void_p(_stream()),
+        sc, float(fill), kind, lo, hi, int(bool(prune)), _stream(),
     )
     return FlashOut(o, lse, m, den)
 
@@ -310,9 +322,10 @@ def flash_fwd_prepared(q, k, v, *, scale: float | None = None, band: Band | None
     fn = getattr(C.CDLL(str(_lib.LIB_PATH)), "pdh_flash_fwd")
     fn.restype = C.c_int
     i64, i32 = C.c_int64, C.c_int
-    args = (_ptr(q), _ptr(k), _ptr(v), _ptr(o), C.c_void_p(None), C.c_void_p(None), _ptr(lse), C.byref(g),
+    vp = C.c_void_p
+    args = (vp(_ptr(q)), vp(_ptr(k)), vp(_ptr(v)), vp(_ptr(o)), vp(None), vp(None), vp(_ptr(lse)), C.byref(g),
             i32(_DT[q.dtype]), C.c_float(sc), C.c_float(fill), i32(kind), i64(lo), i64(hi), i32(int(bool(prune))),
-            C.c_void_p(_stream()))
+            vp(_stream()))
     keep = (q, k, v, o, lse, g)  # the bound pointers' owners live as long as the call
 
     def call():
@@ -331,7 +344,7 @@ def pick_fwd_splits(ninst: int, t: int, s: int, cus: int | None = None) -> int:
     (512 keys); otherwise runs of at least 8 key tiles (256 keys), up to
     three workgroups per CU in all."""
     if cus is None:
-        cus = _lib.lib().pdh_device_cus() or 256
+        cus = _cus()
     blocks = ninst * ((t + 127) // 128)
     ntiles = (s + 31) // 32
     if blocks == 0 or blocks >= 2 * cus or ntiles < 16:
@@ -369,13 +382,13 @@ def flash_bwd(
             raise ValueError(f"{nm} must be contiguous fp32 [batch, heads, rows]")
     if (m is None) != (den is None):
         raise ValueError("pass both m and den, or neither")
-    ws = torch.empty((3,) + tuple(q.shape[:3]), dtype=torch.float32, device=q.device)
+    ws = q.new_empty((3,) + tuple(q.shape[:3]), dtype=torch.float32)
     sc = 1.0 / math.sqrt(q.shape[3]) if scale is None else float(scale)
     kind, (lo, hi) = (PDH_MASK_NONE, (0, 0)) if band is None else (PDH_MASK_BAND, band.c_args())
     _lib.call(
         "pdh_flash_bwd",
         _ptr(q), _ptr(k), _ptr(v), _ptr(o), _ptr(do), _ptr(lse), _ptr(m), _ptr(den), _ptr(dq), _ptr(dk), _ptr(dv),
-        _ptr(ws), C.byref(g), _DT[q.dtype], C.c_float(sc), C.c_float(fill), kind, lo, hi, C.c_void_p(_stream()),
+        _ptr(ws), C.byref(g), _DT[q.dtype], sc, float(fill), kind, lo, hi, _stream(),
     )
     return dq, dk, dv
 
@@ -394,19 +407,19 @@ def attn_decode(
     k / v [B, Hkv, S, D]; every cache row is live."""
     _require_cuda(q, k, v)
     B, Hq, T, D = q.shape
-    o = torch.empty((B, Hq, T, v.shape[3]), dtype=q.dtype, device=q.device)
+    o = q.new_empty((B, Hq, T, v.shape[3]))
     g = _geom(q, k, v, o)
     if nsplit is None:
         nsplit = pick_decode_splits(B * k.shape[1], k.shape[2])
     need = _lib.lib().pdh_attn_decode_workspace(C.byref(g), int(nsplit))
     if workspace is None or workspace.numel() * workspace.element_size() < need:
-        workspace = torch.empty((max(need, 16) + 3) // 4, dtype=torch.float32, device=q.device)
-    lse = torch.empty((B, Hq, T), dtype=torch.float32, device=q.device) if want_lse else None
+        workspace = q.new_empty((max(need, 16) + 3) // 4, dtype=torch.float32)
+    lse = q.new_empty((B, Hq, T), dtype=torch.float32) if want_lse else None
     sc = 1.0 / math.sqrt(D) if scale is None else float(scale)
     _lib.call(
         "pdh_attn_decode",
-        _ptr(q), _ptr(k), _ptr(v), _ptr(o), _ptr(lse), C.byref(g), _DT[q.dtype], C.c_float(sc), int(nsplit),
-        _ptr(workspace), C.c_size_t(workspace.numel() * workspace.element_size()), C.c_void_p(_stream()),
+        _ptr(q), _ptr(k), _ptr(v), _ptr(o), _ptr(lse), C.byref(g), _DT[q.dtype], sc, int(nsplit),
+        _ptr(workspace), workspace.numel() * workspace.element_size(), _stream(),
     )
     return o, lse
 
@@ -432,8 +445,8 @@ def attn_decode_static(
     sc = 1.0 / math.sqrt(q.shape[3]) if scale is None else float(scale)
     _lib.call(
         "pdh_attn_decode_noalloc",
-        _ptr(q), _ptr(k), _ptr(v), _ptr(o), _ptr(lse), C.byref(g), _DT[q.dtype], C.c_float(sc), int(nsplit),
-        C.c_void_p(_stream()),
+        _ptr(q), _ptr(k), _ptr(v), _ptr(o), _ptr(lse), C.byref(g), _DT[q.dtype], sc, int(nsplit),
+        _stream(),
     )
 
 
@@ -465,8 +478,14 @@ def map_chain(prog: _lib.EwProgram, operands: list, out: torch.Tensor) -> torch.
     if out.dtype not in _DT:
         raise ValueError(f"element type {out.dtype} (f32, bf16, f16)")
     _check_views(prog, operands, out, prog.ndim)
-    table = (C.c_void_p * max(1, len(operands)))(*[t.data_ptr() for t in operands])
-    _lib.call("pdh_map_chain", C.byref(prog), table, _ptr(out), _DT[out.dtype], C.c_void_p(_stream()))
+    return map_chain_bound(prog, [t.data_ptr() for t in operands], out)
+
+
+def map_chain_bound(prog: _lib.EwProgram, pointers: list, out: torch.Tensor) -> torch.Tensor:
+    """:func:`map_chain` for a caller whose operands' sizes it has already
+    checked against the program's views: operand i starts at ``pointers[i]``."""
+    table = (C.c_void_p * max(1, len(pointers)))(*pointers)
+    _lib.call("pdh_map_chain", C.byref(prog), table, out.data_ptr(), _DT[out.dtype], _stream())
     return out
 
 
@@ -513,7 +532,7 @@ def contract(a: torch.Tensor, bt: torch.Tensor, k: int, epi: _lib.EwProgram, ope
     table = (C.c_void_p * max(1, len(operands)))(*[t.data_ptr() for t in operands])
     _with_f32_mode(f32_mode, a.dtype, lambda: _lib.call(
         "pdh_contract", _ptr(a), _ptr(bt), B, M, N, int(k), KP, C.byref(epi), table, _ptr(out), _DT[a.dtype],
-        C.c_void_p(_stream()),
+        _stream(),
     ))
     return out
 
@@ -541,12 +560,12 @@ def contract_strided(a: torch.Tensor, a_strides, bt: torch.Tensor, bt_strides, s
     if ksplit == 1:
         call = lambda: _lib.call(  # noqa: E731
             "pdh_contract_strided", _ptr(a), int(a_strides[0]), int(a_strides[1]), _ptr(bt), int(bt_strides[0]),
-            int(bt_strides[1]), B, M, N, Kd, C.byref(epi), table, _ptr(out), _DT[a.dtype], C.c_void_p(_stream()))
+            int(bt_strides[1]), B, M, N, Kd, C.byref(epi), table, _ptr(out), _DT[a.dtype], _stream())
     else:
         call = lambda: _lib.call(  # noqa: E731
             "pdh_contract_strided_ksplit", _ptr(a), int(a_strides[0]), int(a_strides[1]), _ptr(bt),
             int(bt_strides[0]), int(bt_strides[1]), B, M, N, Kd, int(ksplit), C.byref(epi), table, _ptr(out),
-            _DT[a.dtype], C.c_void_p(_stream()))
+            _DT[a.dtype], _stream())
     _with_f32_mode(f32_mode, a.dtype, call)
     return out
 
@@ -576,7 +595,7 @@ def contract_views(a: torch.Tensor, a_strides, bt: torch.Tensor, bt_strides, sha
     sa, sb_ = [int(x) for x in a_strides], [int(x) for x in bt_strides]
     _with_f32_mode(f32_mode, a.dtype, lambda: _lib.call(
         "pdh_contract_views", _ptr(a), *sa, _ptr(bt), *sb_, B, M, N, Kd, int(ksplit), C.byref(epi), table,
-        _ptr(out), _DT[a.dtype], C.c_void_p(_stream())))
+        _ptr(out), _DT[a.dtype], _stream()))
     return out
 
 
@@ -636,7 +655,7 @@ def contract_views_pro(a, a_strides, bt, bt_strides, shape, epi: _lib.EwProgram,
     _with_f32_mode(f32_mode, dt, lambda: _lib.call(
         "pdh_contract_views_pro", pa, sab, sar, sak, progs[0] if progs[0] is not None else null_prog,
         tables[0], pb, sbb, sbr, sbk, progs[1] if progs[1] is not None else null_prog, tables[1],
-        B, M, N, Kd, int(ksplit), C.byref(epi), table, _ptr(out), _DT[dt], C.c_void_p(_stream())))
+        B, M, N, Kd, int(ksplit), C.byref(epi), table, _ptr(out), _DT[dt], _stream()))
     return out
 
 
@@ -692,7 +711,7 @@ def contract_views_rowred(a: torch.Tensor, a_strides, bt: torch.Tensor, bt_strid
     sa, sb_ = [int(x) for x in a_strides], [int(x) for x in bt_strides]
     _with_f32_mode(f32_mode, a.dtype, lambda: _lib.call(
         "pdh_contract_views_rowred", _ptr(a), *sa, _ptr(bt), *sb_, B, M, N, Kd, C.byref(epi), table,
-        _REDUCERS[reducer], _ptr(partials), _DT[a.dtype], C.c_void_p(_stream())))
+        _REDUCERS[reducer], _ptr(partials), _DT[a.dtype], _stream()))
     return partials
 
 
@@ -716,7 +735,7 @@ def reduce_rows(summand: _lib.EwProgram, nk: int, epi: _lib.EwProgram, operands:
         raise ValueError("the epilogue's output view reaches past the output tensor")
     table = (C.c_void_p * max(1, len(operands)))(*[t.data_ptr() for t in operands])
     _lib.call("pdh_reduce_rows_ex", C.byref(summand), int(nk), C.byref(epi), table, len(operands), _ptr(out),
-              _DT[out.dtype], _REDUCERS[reducer], C.c_void_p(_stream()))
+              _DT[out.dtype], _REDUCERS[reducer], _stream())
     return out
 
 
@@ -743,7 +762,7 @@ def scan(x: torch.Tensor, dim: int, f: str = "sum", *, reverse: bool = False,
     outer = math.prod(x.shape[:dim])
     inner = math.prod(x.shape[dim + 1:])
     _lib.call("pdh_scan", _ptr(x), _ptr(y), outer, x.shape[dim], inner, _DT[x.dtype], _SCAN[f],
-              1 if reverse else 0, C.c_void_p(_stream()))
+              1 if reverse else 0, _stream())
     return y
 
 
@@ -751,7 +770,7 @@ def pick_decode_splits(groups: int, s: int, cus: int | None = None) -> int:
     """Splits so the (batch x kv-head x split) grid covers the chip ~8 deep,
     with at least 256 keys per split."""
     if cus is None:
-        cus = _lib.lib().pdh_device_cus() or 256
+        cus = _cus()
     want = max(1, (8 * cus + groups - 1) // groups)
     return int(max(1, min(want, s // 256 if s >= 256 else 1)))
 
@@ -761,6 +780,6 @@ def probe_mfma(a32, b32, a16, b16):
     c32 = torch.empty((32, 32), dtype=torch.float32, device=a32.device)
     c16 = torch.empty((16, 16), dtype=torch.float32, device=a32.device)
     _lib.call(
-        "pdh_probe_mfma", _ptr(a32), _ptr(b32), _ptr(c32), _ptr(a16), _ptr(b16), _ptr(c16), C.c_void_p(_stream())
+        "pdh_probe_mfma", _ptr(a32), _ptr(b32), _ptr(c32), _ptr(a16), _ptr(b16), _ptr(c16), _stream()
     )
     return c32, c16
