@@ -348,6 +348,23 @@ int pdh_contract_views(const void* a, int64_t sa_b, int64_t sa_r, int64_t sa_k, 
                        int64_t sb_r, int64_t sb_k, int64_t batch, int64_t m, int64_t n, int64_t k, int64_t ksplit,
                        const pdh_ew_program* epi, const void* const* operands, void* out, int dtype, void* stream);
 
+/* The 16-bit contraction over operands read in place as views, the
+ * counterpart of pdh_contract_views: each operand has k contiguous (sa_k == 1,
+ * rows at least k apart) or its rows contiguous (sa_r == 1, k at least the
+ * rows apart, their number a multiple of 8: a weight stored [k][n]), strides
+ * multiples of 8 elements, 16-byte aligned bases, k a multiple of 8. Where the
+ * output's tiles cannot fill the chip each entry's k is split over workgroups:
+ * fp32 partial sums go to `ws` (pdh_contract_any_workspace bytes, 0 when no
+ * split; 16-byte aligned) and a second kernel adds them in slice order and
+ * applies the epilogue once. PDH_BF16 / PDH_F16; the epilogue runs on the
+ * runtime-specialized kernels only (PDH_EUNSUPPORTED without them). Replaces
+ * the same reference lowering as pdh_contract_views (fusion.py:159-324). */
+size_t pdh_contract_any_workspace(int64_t batch, int64_t m, int64_t n, int64_t k);
+int pdh_contract_any(const void* a, int64_t sa_b, int64_t sa_r, int64_t sa_k, const void* bt, int64_t sb_b,
+                     int64_t sb_r, int64_t sb_k, int64_t batch, int64_t m, int64_t n, int64_t k,
+                     const pdh_ew_program* epi, const void* const* operands, void* out, int dtype, void* ws,
+                     size_t ws_bytes, void* stream);
+
 /* pdh_contract_views with either operand (or both) computed in the k loop
  * instead of read: pro_a, when not NULL, is an elementwise program over the
  * lattice (batch, m, k) whose value at (b, r, kk) is a[b, r, kk], its LOADs

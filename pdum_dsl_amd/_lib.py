@@ -43,6 +43,8 @@ EXPORTS = (
     "pdh_contract_strided",
     "pdh_contract_strided_ksplit",
     "pdh_contract_views",
+    "pdh_contract_any",
+    "pdh_contract_any_workspace",
     "pdh_contract_views_pro",
     "pdh_contract_views_rowred",
     "pdh_reduce_rows",
@@ -138,6 +140,10 @@ def _declare(lib) -> None:
         "pdh_contract_views": (
             i32, [vp, i64, i64, i64, vp, i64, i64, i64, i64, i64, i64, i64, i64, C.POINTER(EwProgram), C.POINTER(vp),
                   vp, i32, vp]),
+        "pdh_contract_any_workspace": (C.c_size_t, [i64, i64, i64, i64]),
+        "pdh_contract_any": (
+            i32, [vp, i64, i64, i64, vp, i64, i64, i64, i64, i64, i64, i64, C.POINTER(EwProgram), C.POINTER(vp), vp,
+                  i32, vp, C.c_size_t, vp]),
         "pdh_contract_views_pro": (
             i32, [vp, i64, i64, i64, C.POINTER(EwProgram), C.POINTER(vp), vp, i64, i64, i64, C.POINTER(EwProgram),
                   C.POINTER(vp), i64, i64, i64, i64, i64, C.POINTER(EwProgram), C.POINTER(vp), vp, i32, vp]),

@@ -44,16 +44,6 @@ __device__ __forceinline__ void dma4(rsrc_t r, unsigned char* lds, uint32_t voff
 #pragma clang diagnostic pop
 }
 
-// ds_read_b64_tr_b16: in each 16-lane group, lane 4k + c supplies the address
-// of 8 bytes (4 elements); lane i of the group receives element (i % 4) of the
-// chunk addressed by lane 4k + i / 4, for k = 0..3. Pointing lane 4k + c at
-// row k, features 4c..4c+3 of a row-major tile gives lane i the 4 rows' values
-// of feature i: a transposed (k-contiguous) MFMA operand.
-typedef short s16x4_t __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ u32x2 ds_read_tr16(const unsigned char* p) {
-  typedef __attribute__((address_space(3))) s16x4_t lds_s16x4;
-  const s16x4_t v = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(p));
-  return __builtin_bit_cast(u32x2, v);
-}
+// (ds_read_tr16: dev.h)
 
 }  // namespace pdh

@@ -7,6 +7,7 @@
 
 #include "common.h"
 #include "contract_core.h"
+#include "contract_host.h"
 #include "jit.h"
 
 namespace pdh {
@@ -143,6 +144,8 @@ bool reduce_by_columns(const pdh_ew_program& ps, int nk, int nr, int64_t rows) {
 
 // -------------------------------------------------------------- validation
 
+}  // namespace
+
 // A program is checked in full on the host before any launch: opcodes,
 // register numbers, operand slots and dims in range.
 int check_program(const pdh_ew_program* p, int ndim, bool allow_acc, const char* fn) {
@@ -184,6 +187,8 @@ int check_view(const pdh_ew_program* p, const int64_t* stride, const char* fn, c
   return PDH_OK;
 }
 
+namespace {
+
 int dtype_ok(int dtype) { return dtype == PDH_F32 || dtype == PDH_BF16 || dtype == PDH_F16; }
 
 }  // namespace
@@ -214,7 +219,7 @@ extern "C" int pdh_map_chain(const pdh_ew_program* prog, const void* const* oper
   const int64_t nthreads = four ? total / 4 : total;
   const dim3 grid(static_cast<unsigned>((nthreads + 255) / 256));
   uint32_t tot = static_cast<uint32_t>(total);
-  hipFunction_t fns[2];
+  hipFunction_t fns[kJitFns];
   if (jit_get(JitKind::MapChain, *prog, dtype, fns)) {
     pdh_ew_program pa = *prog;
     void* args[] = {&pa, &ops, &out, &tot};
@@ -268,7 +273,7 @@ int contract_launch(ContractArgs ca, const pdh_ew_program* epi, const void* cons
   PDH_REQUIRE((m + 128) * ca.sa_r * esize + ca.kp * ca.sa_k * esize < (int64_t{1} << 31) &&
                   (n + 128) * ca.sb_r * esize + ca.kp * ca.sb_k * esize < (int64_t{1} << 31),
               PDH_EINVAL, "%s: one k slice of a / bt must span under 2 GiB", fn);
-  hipFunction_t fns[2];
+  hipFunction_t fns[kJitFns];
   // operand layouts of the fp32 split kernels: bit 0 a, bit 1 bt rows-contiguous
   // (a computed operand takes the k-contiguous layout)
   const int lay = (ca.sa_k != 1 && !ca.pro_a ? 1 : 0) | (ca.sb_k != 1 && !ca.pro_b ? 2 : 0);
@@ -600,7 +605,7 @@ extern "C" int pdh_reduce_rows_ex(const pdh_ew_program* summand, int nk, const p
   const dim3 grid(static_cast<unsigned>(cols ? (rows + kColOut - 1) / kColOut : (rows + 3) / 4));
   const unsigned threads = cols ? kColOut * kColK : 256;
   int r32 = static_cast<int>(rows);
-  hipFunction_t fns[2];
+  hipFunction_t fns[kJitFns];
   if (jit_get_reduce(*summand, *epi, dtype, fns)) {
     pdh_ew_program a = *summand, b = *epi;
     void* args[] = {&a, &b, &ops, &out, &nk, &r32, &reducer};

@@ -13,7 +13,8 @@
 //                      copied HBM -> LDS by direct buffer loads, double
 //                      buffered; XOR-swizzled 16-byte slots keep the b128
 //                      operand reads conflict-free for 32- and 64-bank LDS;
-//                      a and bt are read through batch and row strides
+//                      a and bt are read through batch and row strides, and
+//                      either may be stored transposed (rows contiguous)
 //   contract_split_body fp32 on the bf16 matrix cores: the same tiles, fp32
 //                      k tiles of 32 loaded to registers, split into two or
 //                      three bf16 planes in LDS, and the cross products of
@@ -121,6 +122,11 @@ __device__ __forceinline__ f32x4 pro_eval4(const ContractPro& pr, const Contract
   const bool rin = row < rows;
   return f32x4{rin ? x[0] : 0.f, rin ? x[1] : 0.f, rin ? x[2] : 0.f, rin ? x[3] : 0.f};
 }
+
+template <bool B>
+struct BoolC {  // a compile-time flag passed to generic lambdas
+  static constexpr bool value = B;
+};
 
 // Element offsets of batch index bb's a and bt rows (the batch entry's, moved
 // to its k slice).
@@ -384,15 +390,16 @@ __device__ __forceinline__ void contract_epilogue(const pdh_ew_program& p, const
     Eval::template run<EPT>(p, ops, DT, c0, acc, res, 1);
     if constexpr (EPT % 4 == 0) {
       const long long o0 = rbase + col0;
-      if (p.out_stride[2] == 1 && (o0 & 3) == 0 && (reinterpret_cast<uintptr_t>(a.out) & 15) == 0) {
-        // runs of four consecutive, aligned outputs: one 16-byte (fp32) or
-        // 8-byte (16-bit) store each; 16-bit runs of eight that start on a
-        // multiple of 8: one 16-byte store each
+      if (p.out_stride[2] == 1) {
+        // runs of consecutive outputs: 16 bytes a store (8 where a 16-bit run of
+        // eight starts between multiples of 8). Rows of an odd length start
+        // anywhere, and the hardware takes those stores too (a vocabulary of
+        // 50257 bf16 logits over 1024 tokens: 215 -> 143 us).
         if constexpr (DT == PDH_F32) {
+          float* o = static_cast<float*>(a.out) + o0;
 #pragma unroll
           for (int q = 0; q < EPT / 4; ++q)
-            *reinterpret_cast<f32x4*>(static_cast<float*>(a.out) + o0 + 4 * q) =
-                f32x4{res[4 * q], res[4 * q + 1], res[4 * q + 2], res[4 * q + 3]};
+            *reinterpret_cast<f32x4u*>(o + 4 * q) = f32x4u{res[4 * q], res[4 * q + 1], res[4 * q + 2], res[4 * q + 3]};
         } else {
           uint16_t* o = static_cast<uint16_t*>(a.out) + o0;
           u32x2 pk[EPT / 4];
@@ -401,13 +408,13 @@ __device__ __forceinline__ void contract_epilogue(const pdh_ew_program& p, const
             const float r4[4] = {res[4 * q], res[4 * q + 1], res[4 * q + 2], res[4 * q + 3]};
             pk[q] = pack4_16<DT>(r4);
           }
-          if (EPT % 8 == 0 && (o0 & 7) == 0) {
+          if constexpr (EPT % 8 == 0) {
 #pragma unroll
             for (int q = 0; q < EPT / 8; ++q)
-              *reinterpret_cast<u32x4*>(o + 8 * q) = u32x4{pk[2 * q][0], pk[2 * q][1], pk[2 * q + 1][0], pk[2 * q + 1][1]};
+              *reinterpret_cast<u32x4h*>(o + 8 * q) = u32x4h{pk[2 * q][0], pk[2 * q][1], pk[2 * q + 1][0], pk[2 * q + 1][1]};
           } else {
 #pragma unroll
-            for (int q = 0; q < EPT / 4; ++q) *reinterpret_cast<u32x2*>(o + 4 * q) = pk[q];
+            for (int q = 0; q < EPT / 4; ++q) *reinterpret_cast<u32x2h*>(o + 4 * q) = u32x2h{pk[q][0], pk[q][1]};
           }
         }
         return;
@@ -552,49 +559,90 @@ __device__ __forceinline__ void contract_store(const ContractArgs& a, const pdh_
   }
 }
 
-template <int DT, int WM, typename Eval>
-__device__ __forceinline__ void contract_mfma_body(const ContractArgs& a, const pdh_ew_program& p,
-                                                   const EwOperands& ops, unsigned char* smem) {
+// The products of a workgroup's tile: acc += a's rows x bt's rows over the
+// batch index's k slice. LAY bit 0: a is rows-contiguous (its row stride is 1
+// and k strided: a transposed tensor), bit 1: bt is (a weight stored [k][n]);
+// otherwise k is contiguous. A k-contiguous operand's tile is BM rows of 64 k
+// values, a rows-contiguous one's 64 k rows of BM values, read transposed by
+// ds_read_b64_tr_b16; both arrive by direct loads of 1 KB. Returns with every
+// wave done with the operand tiles.
+// What bounds it: the loads and the products of a k tile overlap only in part.
+// 4096^3: 129 us, 86 without the loads, 94 without the products; 1024 x 768 x
+// 3072 (64 x 64 tiles, 48 k tiles): 16.5 us, 12.4, 13.3. Eight k tiles in flight,
+// two groups of four waves that split each k tile, and one workgroup of eight
+// waves with four 128-wide tiles in flight measured the same or slower.
+template <int DT, int WM, int LAY>
+__device__ __forceinline__ void contract_mfma_loop(const ContractArgs& a, unsigned char* smem,
+                                                   f32x16 (&acc)[WM / 32][WM / 32], int b, int m0, int n0) {
   constexpr int BM = 2 * WM;          // workgroup tile (rows of a and of bt)
   constexpr int TI = WM / 32;         // 32 x 32 products per wave and dim
   constexpr int TILEB = BM * kRowB;   // LDS bytes per operand tile
-  constexpr int BLK = BM / 8 / 4;     // 8-row direct-load blocks per wave and operand
+  constexpr int BLK = BM / 8 / 4;     // 1 KB direct-load blocks per wave and operand
   constexpr int NS = contract_stages<WM>();
   constexpr int PER_STAGE = 2 * BLK;  // direct loads per wave and k tile
-  const int tid = threadIdx.x, lane = tid & 63, w = wave_id(), r32 = lane & 31, g = lane >> 5;
-  (void)tid;
+  constexpr bool CA = (LAY & 1) != 0, CB = (LAY & 2) != 0;
+  constexpr int PITCH = BM * 2, SLC = BM / 8, RPK = 64 / SLC;  // a rows-contiguous tile: bytes and slots per k row, k rows per block
+  constexpr uint32_t kOOB = 0x80000000u;  // past every buffer's extent: reads as zero
+  static_assert(contract_lds<WM>() >= 2 * NS * TILEB, "operand stages fit the LDS block");
+  const int lane = threadIdx.x & 63, w = wave_id(), r32 = lane & 31, g = lane >> 5;
   const int wy = w >> 1, wx = w & 1;  // the wave's WM x WM quadrant
-  const int per = a.tiles_m * a.tiles_n;
-  const int b = blockIdx.x / per, rest = blockIdx.x % per;
-  const int m0 = (rest / a.tiles_n) * BM, n0 = (rest % a.tiles_n) * BM;
-  const uint32_t rowa = static_cast<uint32_t>(a.sa_r) * 2u, rowbb = static_cast<uint32_t>(a.sb_r) * 2u;
+  int kin = contract_kvalid(a, b) < a.kp ? contract_kvalid(a, b) : a.kp;
+  kin = (kin + 7) & ~7;  // k values of this slice, in whole chunks (the operands are zero between k and there)
+  const uint32_t rowa = static_cast<uint32_t>(CA ? a.sa_k : a.sa_r) * 2u;
+  const uint32_t rowbb = static_cast<uint32_t>(CB ? a.sb_k : a.sb_r) * 2u;
   const uint16_t* abase = static_cast<const uint16_t*>(a.a) + contract_off_a(a, b);
   const uint16_t* bbase = static_cast<const uint16_t*>(a.bt) + contract_off_b(a, b);
-  // the buffers end after the batch slice's last row: rows past m (n) read as zero
-  const rsrc_t ar = make_rsrc(abase, (static_cast<uint32_t>(a.m) - 1u) * rowa + static_cast<uint32_t>(a.kp) * 2u);
-  const rsrc_t br = make_rsrc(bbase, (static_cast<uint32_t>(a.n) - 1u) * rowbb + static_cast<uint32_t>(a.kp) * 2u);
+  // the buffers end after the slice's last row: rows past m (n), or past k, read as zero
+  auto extent = [&](bool c, int rows, uint32_t pitch) {
+    return c ? (static_cast<uint32_t>(kin) - 1u) * pitch + static_cast<uint32_t>(rows) * 2u
+             : (static_cast<uint32_t>(rows) - 1u) * pitch + static_cast<uint32_t>(kin) * 2u;
+  };
+  const rsrc_t ar = make_rsrc(abase, extent(CA, a.m, rowa)), br = make_rsrc(bbase, extent(CB, a.n, rowbb));
 
-  // direct loads: 1 KB = 8 tile rows; lane i -> row i / 8, slot i % 8 holds chunk slot ^ swz(row)
+  // direct loads: 1 KB = 8 tile rows of 64 k values (lane i -> row i / 8, slot i % 8 holds chunk slot ^ swz(row)),
+  // or RPK k rows of BM values (lane i -> row i / SLC, slot i % SLC)
   const int lrow = lane >> 3, slot = lane & 7;
+  int ch[2];
   uint32_t offa[2], offb[2];  // tile-row parity of the 8-row block decides the swizzle of row 8 j + lrow
+  const int crow = lane / SLC, cswz = BM == 128 ? 4 * (crow & 3) : 4 * ((crow >> 1) & 1);
+  const uint32_t cslot = static_cast<uint32_t>(((lane % SLC) ^ cswz) << 4);
 #pragma unroll
   for (int par = 0; par < 2; ++par) {
-    const uint32_t sl = static_cast<uint32_t>((slot ^ swz_gemm(8 * par + lrow)) << 4);
-    offa[par] = lrow * rowa + sl;
-    offb[par] = lrow * rowbb + sl;
+    ch[par] = slot ^ swz_gemm(8 * par + lrow);
+    const uint32_t sl = static_cast<uint32_t>(ch[par] << 4);
+    offa[par] = CA ? crow * rowa + cslot : lrow * rowa + sl;
+    offb[par] = CB ? crow * rowbb + cslot : lrow * rowbb + sl;
   }
-  auto stage = [&](int kt, int buf) {  // stage buf: a tile at 2 buf, bt tile at 2 buf + 1
-    unsigned char* at = smem + (2 * buf) * TILEB;
-    unsigned char* bt = smem + (2 * buf + 1) * TILEB;
-    const uint32_t koff = static_cast<uint32_t>(kt) * kBK * 2u;
+  // This wave's blocks of the next k tile to stage: scalar offsets into the
+  // buffers and LDS, moved on by one add each (the loads of a k tile are
+  // otherwise as much scalar work as the tile has products).
+  uint32_t soa[BLK], sob[BLK], lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(smem)) + w * 1024;
+#pragma unroll
+  for (int i = 0; i < BLK; ++i) {
+    const int blk = 4 * i + w;
+    soa[i] = CA ? static_cast<uint32_t>(RPK * blk) * rowa + static_cast<uint32_t>(m0) * 2u
+                : static_cast<uint32_t>(m0 + 8 * blk) * rowa;
+    sob[i] = CB ? static_cast<uint32_t>(RPK * blk) * rowbb + static_cast<uint32_t>(n0) * 2u
+                : static_cast<uint32_t>(n0 + 8 * blk) * rowbb;
+  }
+  const uint32_t stepa = CA ? kBK * rowa : kBK * 2u, stepb = CB ? kBK * rowbb : kBK * 2u;
+  int sk0 = 0, sbuf = 0;  // the next k tile's first k, its stage
+  auto stage = [&]() __attribute__((always_inline)) {  // stage s: a tile at 2 s, bt tile at 2 s + 1
+    const bool cut = sk0 + kBK > kin;  // the last, ragged k tile
+    const uint32_t lds = lds0 + sbuf * (2 * TILEB);
 #pragma unroll
     for (int i = 0; i < BLK; ++i) {
-      const int blk = 4 * i + w;  // BM / 8 blocks of 8 rows per operand tile
-      dma16(ar, at + blk * 1024, offa[blk & 1], static_cast<uint32_t>(m0 + 8 * blk) * rowa + koff);
-      dma16(br, bt + blk * 1024, offb[blk & 1], static_cast<uint32_t>(n0 + 8 * blk) * rowbb + koff);
+      const int par = w & 1;
+      const bool out = cut && sk0 + 8 * ch[par] >= kin;
+      dma16_at(ar, lds + i * 4096, CA ? offa[0] : (out ? kOOB : offa[par]), soa[i]);
+      dma16_at(br, lds + TILEB + i * 4096, CB ? offb[0] : (out ? kOOB : offb[par]), sob[i]);
+      soa[i] += stepa;
+      sob[i] += stepb;
     }
+    sk0 += kBK;
+    sbuf = sbuf + 1 == NS ? 0 : sbuf + 1;
   };
-  // operand reads: row (WM q + 32 t + r32) of a tile, chunk 2 ks + g
+  // operand reads. k-contiguous: row (WM q + 32 t + r32) of a tile, chunk 2 ks + g
   int rd[TI][4];
 #pragma unroll
   for (int t = 0; t < TI; ++t)
@@ -603,36 +651,57 @@ __device__ __forceinline__ void contract_mfma_body(const ContractArgs& a, const 
       const int row = 32 * t + r32;  // + WM q: a multiple of 16 rows, so the swizzle is unchanged
       rd[t][ks] = row * kRowB + (((2 * ks + g) ^ swz_gemm(row)) << 4);
     }
+  // rows-contiguous: 16-lane group G reads k rows 16 ks + 8 (G / 2) + 0..3 (and + 4) of columns WM q + 32 t + 16 (G % 2) ..+15
+  const int i4 = (lane >> 2) & 3, c4 = lane & 3, G = lane >> 4;
+  const int tswz = BM == 128 ? 4 * i4 : 4 * (i4 >> 1);
+  auto tr_off = [&](int q, int t) {
+    const int s = WM / 8 * q + 4 * t + 2 * (G & 1) + (c4 >> 1);
+    return (8 * (G >> 1) + i4) * PITCH + ((s ^ tswz) << 4) + ((c4 & 1) << 3);
+  };
+  int tra[TI], trb[TI];
+#pragma unroll
+  for (int t = 0; t < TI; ++t) {
+    tra[t] = tr_off(wy, t);
+    trb[t] = tr_off(wx, t);
+  }
+  auto frag = [&](auto c_c, const unsigned char* tile, int q, const int (&rdt)[4], int trt, int ks)
+      __attribute__((always_inline)) {
+        if constexpr (decltype(c_c)::value) {
+          const u32x2 lo = ds_read_tr16(tile + trt + 16 * ks * PITCH);
+          const u32x2 hi = ds_read_tr16(tile + trt + (16 * ks + 4) * PITCH);
+          return u32x4{lo.x, lo.y, hi.x, hi.y};
+        } else {
+          return *reinterpret_cast<const u32x4*>(tile + WM * q * kRowB + rdt[ks]);
+        }
+      };
 
-  f32x16 acc[TI][TI];
 #pragma unroll
   for (int i = 0; i < TI; ++i)
 #pragma unroll
     for (int j = 0; j < TI; ++j) acc[i][j] = f32x16{};
 
-  const int nkt = a.kp / kBK;
-  static_assert(contract_lds<WM>() >= 2 * NS * TILEB, "operand stages fit the LDS block");
+  const int nkt = (kin + kBK - 1) / kBK;
 #pragma unroll
   for (int s = 0; s < NS - 1; ++s)
-    if (s < nkt) stage(s, s);
-  for (int kt = 0; kt < nkt; ++kt) {
-    const int buf = kt % NS;
+    if (s < nkt) stage();
+  int buf = 0;  // kt % NS
+  for (int kt = 0; kt < nkt; ++kt, buf = buf + 1 == NS ? 0 : buf + 1) {
     // tile kt has landed when at most the NS - 2 later tiles' loads are outstanding
     if (kt + NS - 2 < nkt)
       wait_vmcnt<(NS - 2) * PER_STAGE>();
     else
       wait_vmcnt0();
     __syncthreads();  // every wave's loads of tile kt are done; everyone finished tile kt - 1
-    if (kt + NS - 1 < nkt) stage(kt + NS - 1, (kt + NS - 1) % NS);
-    const unsigned char* at = smem + (2 * buf) * TILEB + WM * wy * kRowB;
-    const unsigned char* bt = smem + (2 * buf + 1) * TILEB + WM * wx * kRowB;
+    if (kt + NS - 1 < nkt) stage();
+    const unsigned char* at = smem + (2 * buf) * TILEB;
+    const unsigned char* bt = smem + (2 * buf + 1) * TILEB;
     u32x4 af[4][TI], bf[4][TI];
 #pragma unroll
     for (int ks = 0; ks < 4; ++ks)
 #pragma unroll
       for (int t = 0; t < TI; ++t) {
-        af[ks][t] = *reinterpret_cast<const u32x4*>(at + rd[t][ks]);
-        bf[ks][t] = *reinterpret_cast<const u32x4*>(bt + rd[t][ks]);
+        af[ks][t] = frag(BoolC<CA>{}, at, wy, rd[t], tra[t], ks);
+        bf[ks][t] = frag(BoolC<CB>{}, bt, wx, rd[t], trb[t], ks);
       }
     __builtin_amdgcn_s_setprio(1);
 #pragma unroll
@@ -646,7 +715,85 @@ __device__ __forceinline__ void contract_mfma_body(const ContractArgs& a, const 
   }
   wait_vmcnt0();
   __syncthreads();  // every wave is done with the operand tiles
-  contract_store<DT, WM, Eval>(a, p, ops, smem, acc, b, m0, n0);
+}
+
+// A workgroup's tile. XCD x (workgroups go round-robin over the eight) takes a
+// contiguous run of an order that walks groups of eight tile rows column by
+// column, so its L2 serves each bt panel to the whole group, and a k slice's
+// operands to its tiles (against row order, 1024 x 50257 x 768: 143 -> 107 us;
+// 458 x 320 x 6144 in six slices: 16.1 -> 12.7; 8192 x 3072 x 768: 54 -> 50; the
+// other shapes measured, 1024 x 768 x 768 to 4096^3, within 3%; groups of four
+// rows within 3% of eight).
+struct ContractTile {
+  int b, tm, tn;
+};
+__device__ __forceinline__ ContractTile contract_tile(const ContractArgs& a) {
+  const int per = a.tiles_m * a.tiles_n;
+  const int total = gridDim.x, q = total >> 3, r = total & 7, x = blockIdx.x & 7;
+  const int pos = x * q + (x < r ? x : r) + (blockIdx.x >> 3);
+  const int b = pos / per, in_b = pos % per;
+  constexpr int GR = 8;
+  const int grp = in_b / (GR * a.tiles_n), left = a.tiles_m - grp * GR, rows = left < GR ? left : GR;
+  const int in = in_b - grp * GR * a.tiles_n;
+  return ContractTile{b, grp * GR + in % rows, in / rows};
+}
+
+template <int DT, int WM, typename Eval, int LAY = 0>
+__device__ __forceinline__ void contract_mfma_body(const ContractArgs& a, const pdh_ew_program& p,
+                                                   const EwOperands& ops, unsigned char* smem) {
+  constexpr int BM = 2 * WM;
+  const ContractTile t = contract_tile(a);
+  f32x16 acc[WM / 32][WM / 32];
+  contract_mfma_loop<DT, WM, LAY>(a, smem, acc, t.b, t.tm * BM, t.tn * BM);
+  contract_store<DT, WM, Eval>(a, p, ops, smem, acc, t.b, t.tm * BM, t.tn * BM);
+}
+
+// A split contraction's partial sums: the fp32 accumulators of batch index b
+// (entry, k slice) as they stand, to ws[b][m][n].
+template <int DT, int LAY>
+__device__ __forceinline__ void contract_part_body(const ContractArgs& a, float* ws, unsigned char* smem) {
+  const ContractTile t = contract_tile(a);
+  const int m0 = t.tm * 64, n0 = t.tn * 64;
+  f32x16 acc[1][1];
+  contract_mfma_loop<DT, 32, LAY>(a, smem, acc, t.b, m0, n0);
+  const int lane = threadIdx.x & 63, w = wave_id();
+  const int col = n0 + 32 * (w & 1) + (lane & 31), row0 = m0 + 32 * (w >> 1) + 4 * (lane >> 5);
+  if (col >= a.n) return;
+  float* o = ws + static_cast<long long>(t.b) * a.m * a.n + col;
+#pragma unroll
+  for (int v = 0; v < 16; ++v) {
+    const int row = row0 + 8 * (v >> 2) + (v & 3);
+    if (row < a.m) o[static_cast<long long>(row) * a.n] = acc[0][0][v];
+  }
+}
+
+// The finish of a split contraction: each output's slices summed in order,
+// then the epilogue and the one rounding. Four consecutive columns per lane.
+template <int DT, typename Eval>
+__device__ __forceinline__ void contract_finish_body(const ContractArgs& a, const pdh_ew_program& p,
+                                                     const EwOperands& ops, const float* ws) {
+  const int quads = (a.n + 3) >> 2;
+  const long long idx = static_cast<long long>(blockIdx.x) * 256 + threadIdx.x;
+  const int col = static_cast<int>(idx % quads) * 4;
+  const long long rr = idx / quads;
+  const int row = static_cast<int>(rr % a.m), e = static_cast<int>(rr / a.m);
+  if (e >= a.batch / a.ksplit) return;
+  const long long plane = static_cast<long long>(a.m) * a.n;
+  const float* src = ws + static_cast<long long>(e) * a.ksplit * plane + static_cast<long long>(row) * a.n + col;
+  float acc[4] = {0.f, 0.f, 0.f, 0.f};
+  if (col + 4 <= a.n) {
+    for (int s = 0; s < a.ksplit; ++s) {
+      const f32x4 x = *reinterpret_cast<const f32x4u*>(src + s * plane);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) acc[j] += x[j];
+    }
+  } else {
+    for (int s = 0; s < a.ksplit; ++s)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (col + j < a.n) acc[j] += src[s * plane + j];
+  }
+  contract_epilogue<DT, 4, Eval>(p, ops, a, e, row, col, acc);
 }
 
 // One 64 x 64 block (rows m0.., columns n0..) of batch b by fp32 VALU fma,
@@ -773,10 +920,6 @@ constexpr int split_lds() {
 // operand and (rows 4 q + c, q = 8 w .. 8 w + 7, all 8 chunks) for a
 // rows-contiguous one.
 __device__ __forceinline__ int swz_split(int r) { return (r >> 2) & 3; }
-template <bool B>
-struct BoolC {  // a compile-time flag passed to generic lambdas
-  static constexpr bool value = B;
-};
 template <typename T>
 struct TypeC {  // a type passed to generic lambdas
   using type = T;

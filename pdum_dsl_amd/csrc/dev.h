@@ -17,6 +17,9 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 // four floats at any 4-byte boundary: one global_load_dwordx4 / store (the
 // hardware takes dword-aligned multi-dword accesses)
 typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+// runs of 16-bit values at any 2-byte boundary
+typedef uint32_t u32x4h __attribute__((ext_vector_type(4), aligned(2)));
+typedef uint32_t u32x2h __attribute__((ext_vector_type(2), aligned(2)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
@@ -118,14 +121,29 @@ __device__ __forceinline__ rsrc_t make_rsrc(const void* base, uint32_t bytes) {
 // wave-uniform). Inline asm keeps the compiler's wait-count pass from making
 // every later LDS read wait for it: callers wait with s_waitcnt vmcnt(0) and a
 // barrier before reading the tile.
-__device__ __forceinline__ void dma16(rsrc_t r, unsigned char* lds, uint32_t voff, uint32_t soff) {
-  // the low 32 bits of a generic LDS address are its LDS offset (no address-space cast needed)
-  const uint32_t m0 = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(reinterpret_cast<uintptr_t>(lds)));
+__device__ __forceinline__ void dma16_at(rsrc_t r, uint32_t lds, uint32_t voff, uint32_t soff) {
+  const uint32_t m0 = __builtin_amdgcn_readfirstlane(lds);
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"  // m0 is reserved: listed so the compiler knows it changes
   asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(m0), "v"(voff), "s"(r), "s"(soff)
                : "memory", "m0");
 #pragma clang diagnostic pop
+}
+__device__ __forceinline__ void dma16(rsrc_t r, unsigned char* lds, uint32_t voff, uint32_t soff) {
+  // the low 32 bits of a generic LDS address are its LDS offset (no address-space cast needed)
+  dma16_at(r, static_cast<uint32_t>(reinterpret_cast<uintptr_t>(lds)), voff, soff);
+}
+
+// ds_read_b64_tr_b16: in each 16-lane group, lane 4k + c supplies the address
+// of 8 bytes (4 elements); lane i of the group receives element (i % 4) of the
+// chunk addressed by lane 4k + i / 4, for k = 0..3. Pointing lane 4k + c at
+// row k, features 4c..4c+3 of a row-major tile gives lane i the 4 rows' values
+// of feature i: a transposed (k-contiguous) MFMA operand.
+typedef short s16x4_t __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ u32x2 ds_read_tr16(const unsigned char* p) {
+  typedef __attribute__((address_space(3))) s16x4_t lds_s16x4;
+  const s16x4_t v = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(p));
+  return __builtin_bit_cast(u32x2, v);
 }
 
 // s_waitcnt vmcnt(0) (expcnt / lgkmcnt left at their maxima), issued through

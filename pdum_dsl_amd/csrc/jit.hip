@@ -33,7 +33,7 @@ std::atomic<int64_t> g_compiled{0}, g_launched{0}, g_failed{0};
 
 struct Entry {
   hipModule_t mod = nullptr;
-  hipFunction_t fn[2] = {nullptr, nullptr};
+  hipFunction_t fn[kJitFns] = {};
   bool ok = false;
 };
 std::mutex g_mu;
@@ -76,13 +76,12 @@ std::string request_key(char what, int dev, int dt, int lay, int red) {
 }
 
 // The entry of request `key` into fns; false when there is none (or the interpreter runs it). known: whether there is one.
-bool find_request(const std::string& key, hipFunction_t fns[2], bool* known) {
+bool find_request(const std::string& key, hipFunction_t fns[kJitFns], bool* known) {
   std::lock_guard<std::mutex> lock(g_mu);
   const auto it = g_by_request.find(key);
   *known = it != g_by_request.end();
   if (!*known || !it->second->ok) return false;
-  fns[0] = it->second->fn[0];
-  fns[1] = it->second->fn[1];
+  for (int i = 0; i < kJitFns; ++i) fns[i] = it->second->fn[i];
   return true;
 }
 
@@ -220,12 +219,22 @@ std::string kernels_src(JitKind kind, int dt, int lay, int red) {
            "smem[pdh::split_lds<32, " + ns + ">()]; pdh::contract_split_body<PDH_F32, 32, " + nl +
            ", pdh::GenEval" + rd + ">(a, p, ops, smem); }\n";
   }
-  return "extern \"C\" __global__ __launch_bounds__(256, 2) void pdh_jit_k0(pdh::ContractArgs a, pdh_ew_program p, "
-         "pdh::EwOperands ops) { __shared__ __attribute__((aligned(1024))) unsigned char "
-         "smem[pdh::contract_lds<64>()]; pdh::contract_mfma_body<" + D + ", 64, pdh::GenEval>(a, p, ops, smem); }\n"
-         "extern \"C\" __global__ __launch_bounds__(256, 2) void pdh_jit_k1(pdh::ContractArgs a, pdh_ew_program p, "
-         "pdh::EwOperands ops) { __shared__ __attribute__((aligned(1024))) unsigned char "
-         "smem[pdh::contract_lds<32>()]; pdh::contract_mfma_body<" + D + ", 32, pdh::GenEval>(a, p, ops, smem); }\n";
+  // 16-bit: 128 x 128 tiles, 64 x 64 tiles, the finish of a k split
+  const std::string args = "(pdh::ContractArgs a, pdh_ew_program p, pdh::EwOperands ops";
+  auto tile = [&](const char* name, const std::string& wm) {
+    return std::string("extern \"C\" __global__ __launch_bounds__(256, 2) void ") + name + args +
+           ") { __shared__ __attribute__((aligned(1024))) unsigned char smem[pdh::contract_lds<" + wm +
+           ">()]; pdh::contract_mfma_body<" + D + ", " + wm + ", pdh::GenEval" +
+           (lay != 0 ? ", " + std::to_string(lay) : "") + ">(a, p, ops, smem); }\n";
+  };
+  return tile("pdh_jit_k0", "64") + tile("pdh_jit_k1", "32") +
+         "extern \"C\" __global__ __launch_bounds__(256) void pdh_jit_k2" + args + ", const float* ws) { "
+         "pdh::contract_finish_body<" + D + ", pdh::GenEval>(a, p, ops, ws); }\n";
+}
+
+// Kernels in a contraction's module.
+int contract_kernels(JitKind kind, int dt) {
+  return kind == JitKind::MapChain ? 2 : (dt != PDH_F32 ? 3 : (f32_contract_mode() != 0 ? 2 : 1));
 }
 
 bool compile_code(const std::string& src, std::vector<char>* code, std::string* err) {
@@ -309,17 +318,19 @@ std::string pro_source(const pdh_ew_program& pe, const pdh_ew_program* pa, const
   return s + k;
 }
 
-bool compile(const std::string& src, bool two, Entry* out, std::string* err) {
+bool compile(const std::string& src, int count, Entry* out, std::string* err) {
   std::vector<char> code;
   if (!compile_code(src, &code, err)) return false;
   if (hipModuleLoadData(&out->mod, code.data()) != hipSuccess) {
     *err = "hipModuleLoadData failed";
     return false;
   }
-  if (hipModuleGetFunction(&out->fn[0], out->mod, "pdh_jit_k0") != hipSuccess ||
-      (two && hipModuleGetFunction(&out->fn[1], out->mod, "pdh_jit_k1") != hipSuccess)) {
-    *err = "hipModuleGetFunction failed";
-    return false;
+  for (int i = 0; i < count; ++i) {
+    const std::string name = "pdh_jit_k" + std::to_string(i);
+    if (hipModuleGetFunction(&out->fn[i], out->mod, name.c_str()) != hipSuccess) {
+      *err = "hipModuleGetFunction failed";
+      return false;
+    }
   }
   return true;
 }
@@ -339,14 +350,14 @@ bool jit_enabled() {
 namespace {
 
 // The entry of `src` (compiled on its first request) into fns, kept under `key` for the next one.
-bool get(const std::string& key, int dev, const std::string& src, bool two, hipFunction_t fns[2]) {
+bool get(const std::string& key, int dev, const std::string& src, int count, hipFunction_t fns[kJitFns]) {
   const std::string skey = std::to_string(dev) + "|" + src;
   std::lock_guard<std::mutex> lock(g_mu);
   auto it = g_cache.find(skey);
   if (it == g_cache.end()) {
     Entry e;
     std::string err;
-    e.ok = compile(src, two, &e, &err);
+    e.ok = compile(src, count, &e, &err);
     if (e.ok)
       ++g_compiled;
     else {
@@ -358,17 +369,15 @@ bool get(const std::string& key, int dev, const std::string& src, bool two, hipF
   }
   g_by_request.emplace(key, &it->second);
   if (!it->second.ok) return false;
-  fns[0] = it->second.fn[0];
-  fns[1] = it->second.fn[1];
+  for (int i = 0; i < kJitFns; ++i) fns[i] = it->second.fn[i];
   return true;
 }
 
 }  // namespace
 
-// The specialized kernel(s) for program p: fn[0] and fn[1] (the one-element
-// map-chain variant; the 64 x 64-tile contraction), or false when the
+// The specialized kernels for program p (jit.h), or false when the
 // interpreter must run it.
-bool jit_get(JitKind kind, const pdh_ew_program& p, int dt, hipFunction_t fns[2], int lay, int red) {
+bool jit_get(JitKind kind, const pdh_ew_program& p, int dt, hipFunction_t fns[kJitFns], int lay, int red) {
   if (!jit_enabled()) return false;
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess) return false;
@@ -378,12 +387,12 @@ bool jit_get(JitKind kind, const pdh_ew_program& p, int dt, hipFunction_t fns[2]
   const bool found = find_request(key, fns, &known);
   return known ? found
                : get(key, dev, full_source(kind, p, dt, lay, red),
-                     kind == JitKind::MapChain || dt != PDH_F32 || f32_contract_mode() != 0, fns);
+                     contract_kernels(kind, dt), fns);
 }
 
 // The specialized row-reduce kernels for (summand, epilogue): fns[0] one
 // wave per output, fns[1] the column variant; or false.
-bool jit_get_reduce(const pdh_ew_program& ps, const pdh_ew_program& pe, int dt, hipFunction_t fns[2]) {
+bool jit_get_reduce(const pdh_ew_program& ps, const pdh_ew_program& pe, int dt, hipFunction_t fns[kJitFns]) {
   if (!jit_enabled()) return false;
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess) return false;
@@ -392,13 +401,13 @@ bool jit_get_reduce(const pdh_ew_program& ps, const pdh_ew_program& pe, int dt, 
   key_program(key, pe);
   bool known;
   const bool found = find_request(key, fns, &known);
-  return known ? found : get(key, dev, reduce_source(ps, pe, dt), true, fns);
+  return known ? found : get(key, dev, reduce_source(ps, pe, dt), 2, fns);
 }
 
 // The fp32 prologue kernels specialized for (epilogue, prologues): fns[0] the
 // 128 x 128-tile kernel (or the VALU one in fp32 mode 0), fns[1] the
 // 64 x 64-tile one; or false.
-bool jit_get_pro(const pdh_ew_program& pe, const pdh_ew_program* pa, const pdh_ew_program* pb, hipFunction_t fns[2],
+bool jit_get_pro(const pdh_ew_program& pe, const pdh_ew_program* pa, const pdh_ew_program* pb, hipFunction_t fns[kJitFns],
                  int lay, int dt) {
   if (!jit_enabled()) return false;
   int dev = 0;
@@ -409,7 +418,8 @@ bool jit_get_pro(const pdh_ew_program& pe, const pdh_ew_program* pa, const pdh_e
   if (pb != nullptr) key_program(key, *pb);
   bool known;
   const bool found = find_request(key, fns, &known);
-  return known ? found : get(key, dev, pro_source(pe, pa, pb, lay, dt), dt != PDH_F32 || f32_contract_mode() != 0, fns);
+  return known ? found : get(key, dev, pro_source(pe, pa, pb, lay, dt),
+                           dt != PDH_F32 || f32_contract_mode() != 0 ? 2 : 1, fns);
 }
 
 void jit_count_launch() { ++g_launched; }

@@ -313,6 +313,72 @@ def with_slots(prog, first: int, total: int):
     return new
 
 
+_CUS = 256  # MI355X compute units
+
+
+def _big_tiles(Bs, M, N, kc=64 * 64):
+    """The launcher's tile choice (contract_launch in contract.hip): 128 x 128
+    workgroup tiles when they give every compute unit one, neither output side
+    is 64 or under and a workgroup's k (kc columns) is over 128; 64 x 64
+    otherwise."""
+    return Bs * -(-M // 128) * -(-N // 128) >= _CUS and M > 64 and N > 64 and kc > 128
+
+
+# Microseconds per 64-column k tile of one workgroup of the fp32 split kernel
+# on MI355X, by workgroups resident on a compute unit: 64 x 64 tiles (up to
+# five resident), 128 x 128 tiles (two; one alone runs a little faster).
+_SMALL_STEP = {1: 1.7, 2: 2.0, 3: 2.7, 4: 3.4, 5: 4.2}
+_BIG_STEP2, _BIG_STEP1 = 5.0, 4.0
+
+
+def _ksplit_est(B, M, N, kt, S):
+    """Estimated microseconds of an fp32 contraction of B (M x N) outputs over
+    kt 64-column k tiles run as S k slices: the busiest compute unit's tiles at
+    the measured per-tile rates, plus a fixed 4 us, plus the pass that adds
+    the S partial planes (S + 1 planes of HBM traffic at 5 TB/s)."""
+    kc = -(-kt // S)
+    if _big_tiles(B * S, M, N, 64 * kc):
+        per = -(-(B * S * -(-M // 128) * -(-N // 128)) // _CUS)
+        t = (per // 2) * kc * _BIG_STEP2 + (per % 2) * kc * _BIG_STEP1
+    else:
+        per = -(-(B * S * -(-M // 64) * -(-N // 64)) // _CUS)
+        t = (per // 5) * kc * _SMALL_STEP[5] + (kc * _SMALL_STEP[per % 5] if per % 5 else 0.0)
+    fin = (S + 1) * B * M * N * 4 / 5e6 if S > 1 else 0.0
+    return 4.0 + t + fin
+
+
+def _ksplit_order(B, M, N, kt):
+    """k slice counts (1..16, none empty, each of at least two k tiles) for
+    an fp32 contraction, cheapest first under :func:`_ksplit_est`, a model
+    fitted to measured times of the gpt2 gradient's contractions on MI355X."""
+    cands = [S for S in range(1, 17) if (S - 1) * -(-kt // S) < kt and (S == 1 or -(-kt // S) >= 2)]
+    return sorted(cands, key=lambda S: (_ksplit_est(B, M, N, kt, S), S))
+
+
+def pick_ksplit(epi: L.EwProgram, B: int, M: int, N: int, kt: int) -> tuple:
+    """(S, partial, finish) for an fp32 contraction over ``kt`` 64-column k
+    tiles whose epilogue is ``epi``: the cheapest slice count under the cost
+    model whose sum fits one map-chain program, the identity program of the
+    [B * S, M, N] partial sums and the program that adds them in order and
+    applies the epilogue; (1, None, None) for no split."""
+    if kt < 4:
+        return 1, None, None
+    for S in _ksplit_order(B, M, N, kt):
+        if S == 1:
+            return 1, None, None
+        fin = splitk_sum(epi, S, (S * M * N, N, 1))
+        if fin is not None:
+            break
+    else:
+        return 1, None, None
+    ident = L.EwProgram()
+    ident.n_insns, ident.n_operands, ident.ndim, ident.out_reg = 1, 0, 3, 0
+    for d, (ext, st) in enumerate(zip((B * S, M, N), (M * N, N, 1))):
+        ident.shape[d], ident.out_stride[d] = ext, st
+    ident.insns[0].op = L.EW["ACC"]
+    return S, ident, fin
+
+
 def splitk_sum(prog, S: int, plane_strides=None):
     """The epilogue program ``prog`` (which reads the contraction's sum with
     ACC) rewritten to read that sum as the total of S partial planes: slots

@@ -51,13 +51,13 @@ from dataclasses import dataclass, field
 
 from . import _lib as L
 from . import ewprog
+from .ewprog import _big_tiles, _ksplit_est, _ksplit_order  # noqa: F401  (the fp32 k-split model)
 from .hip_tile import Untranslatable, recognize_layernorm
 from .tl.dialect import OPS
 from .tl.fusion import contract_core, forest_is_closed, match_contraction_epilogue, match_softmax, plan_region
 from .tl.ir import Builder, Dim, Region, walk
 
 _TORCH_DT = {"f32": "float32", "bf16": "bfloat16", "f16": "float16"}
-_CUS = 256  # MI355X compute units
 
 
 def _torch():
@@ -97,45 +97,6 @@ def _strided_view(tt, riders, rows, kd):
     row = st[rows[-1]] if rows else 0
     batch = st[riders[0]] if riders else 0
     return (batch, row)
-
-
-def _big_tiles(Bs, M, N, kc=64 * 64):
-    """The launcher's tile choice (contract_launch in contract.hip): 128 x 128
-    workgroup tiles when they give every compute unit one, neither output side
-    is 64 or under and a workgroup's k (kc columns) is over 128; 64 x 64
-    otherwise."""
-    return Bs * -(-M // 128) * -(-N // 128) >= _CUS and M > 64 and N > 64 and kc > 128
-
-
-# Microseconds per 64-column k tile of one workgroup of the fp32 split kernel
-# on MI355X, by workgroups resident on a compute unit: 64 x 64 tiles (up to
-# five resident), 128 x 128 tiles (two; one alone runs a little faster).
-_SMALL_STEP = {1: 1.7, 2: 2.0, 3: 2.7, 4: 3.4, 5: 4.2}
-_BIG_STEP2, _BIG_STEP1 = 5.0, 4.0
-
-
-def _ksplit_est(B, M, N, kt, S):
-    """Estimated microseconds of an fp32 contraction of B (M x N) outputs over
-    kt 64-column k tiles run as S k slices: the busiest compute unit's tiles at
-    the measured per-tile rates, plus a fixed 4 us, plus the pass that adds
-    the S partial planes (S + 1 planes of HBM traffic at 5 TB/s)."""
-    kc = -(-kt // S)
-    if _big_tiles(B * S, M, N, 64 * kc):
-        per = -(-(B * S * -(-M // 128) * -(-N // 128)) // _CUS)
-        t = (per // 2) * kc * _BIG_STEP2 + (per % 2) * kc * _BIG_STEP1
-    else:
-        per = -(-(B * S * -(-M // 64) * -(-N // 64)) // _CUS)
-        t = (per // 5) * kc * _SMALL_STEP[5] + (kc * _SMALL_STEP[per % 5] if per % 5 else 0.0)
-    fin = (S + 1) * B * M * N * 4 / 5e6 if S > 1 else 0.0
-    return 4.0 + t + fin
-
-
-def _ksplit_order(B, M, N, kt):
-    """k slice counts (1..16, none empty, each of at least two k tiles) for
-    an fp32 contraction, cheapest first under :func:`_ksplit_est`, a model
-    fitted to measured times of the gpt2 gradient's contractions on MI355X."""
-    cands = [S for S in range(1, 17) if (S - 1) * -(-kt // S) < kt and (S == 1 or -(-kt // S) >= 2)]
-    return sorted(cands, key=lambda S: (_ksplit_est(B, M, N, kt, S), S))
 
 
 def _view3(tt, riders, rows, kd):
@@ -238,6 +199,45 @@ def _under_renames(n):
     while n.op == "tl.rename":
         n = n.args[0]
     return n
+
+
+def _chains_as_epilogues(plan, region: Region):
+    """``plan`` with each map-chain carve that alone reads one GEMM-shaped
+    contraction carve merged into it, as its epilogue (gpt2's gelu(x w + b)
+    before the down projection: two launches and a round trip of the wide
+    activation less). The partition keeps them apart because the bias
+    broadcast onto the sum counts as a second reader of it."""
+    from .tl.partition import Carve, extract
+
+    y = region.body[-1].args[0]
+    outputs = {id(x) for x in (y.args if y.op == "core.tuple" else (y,))}
+    carves = list(plan.carves)
+    for chain in plan.carves:
+        if chain.root is None or chain.artifacts or chain.group.template != "map-chain":
+            continue
+        feeds = [c for c in carves if c.root is not None and c.group.template == "contraction-epilogue"
+                 and not c.artifacts and any(b is c.root for b in chain.bounds)]
+        if len(feeds) != 1 or id(feeds[0].root) in outputs:
+            continue
+        mm = feeds[0]
+        if any(b is mm.root for c in carves if c is not chain for b in c.bounds):
+            continue
+        stop = {id(b) for c in (chain, mm) for b in c.bounds if b is not mm.root}
+        members, stack = {}, [chain.root]
+        while stack:
+            n = stack.pop()
+            if id(n) in members or id(n) in stop or n.op == "core.param":
+                continue
+            members[id(n)] = n
+            stack.extend(n.args)
+        kernel, bounds = extract((chain.root,), members)
+        m = match_contraction_epilogue(kernel)
+        if m is None or m["shape"] != "gemm":
+            continue
+        group = plan_region(kernel).groups[0]
+        merged = Carve(kernel, group, mm.nodes + chain.nodes, chain.root.op, chain.root, bounds, ())
+        carves = [merged if c is chain else c for c in carves if c is not mm]
+    return type(plan)(tuple(carves), plan.interior)
 
 
 def _band_has_empty_row(T: int, S: int, lo, hi) -> bool:
@@ -809,8 +809,8 @@ class PlanExecutor:
         from .tl.partition import plan_model
 
         sub = _yielding(k, node)
-        nested = PlanExecutor(plan_model(sub, dissolve=False), sub, self.dtype, _shared=(self._packs, self._static),
-                              f32_contract=self.f32_contract)
+        nested = PlanExecutor(_chains_as_epilogues(plan_model(sub, dissolve=False), sub), sub, self.dtype,
+                              _shared=(self._packs, self._static), f32_contract=self.f32_contract)
         self.nested.append(nested)
 
         def run(vals):
@@ -1066,21 +1066,8 @@ class PlanExecutor:
         # (whole 64-column tiles, the last ragged) as S workgroups per tile
         # (pdh_contract_views: partial sums into an fp32 workspace
         # [B][S][M][N]), and a map chain adds the slices in order and applies
-        # the epilogue; S is the cheapest under the cost model whose sum fits
-        # one map-chain program.
-        S, fin, ident = 1, None, None
-        if views and KP // 64 >= 4 and rowred is None:
-            for pick in _ksplit_order(B, M, N, KP // 64):
-                fin = ewprog.splitk_sum(prog, pick, (pick * M * N, N, 1)) if pick > 1 else None
-                if pick == 1 or fin is not None:
-                    break
-            if fin is not None:
-                S = pick
-                ident = L.EwProgram()
-                ident.n_insns, ident.n_operands, ident.ndim, ident.out_reg = 1, 0, 3, 0
-                for d, (ext, st) in enumerate(zip((B * S, M, N), (M * N, N, 1))):
-                    ident.shape[d], ident.out_stride[d] = ext, st
-                ident.insns[0].op = L.EW["ACC"]
+        # the epilogue. (16-bit ones split inside pdh_contract_any.)
+        S, ident, fin = ewprog.pick_ksplit(prog, B, M, N, KP // 64) if views and rowred is None else (1, None, None)
 
         def build(p, vals, dt):
             torch = _torch()
@@ -1158,6 +1145,9 @@ class PlanExecutor:
 
                 K.contract_views_pro(None, None, None, None, (B, M, N, Kx), prog, [vals[i] for i in eslots], out,
                                      pro_a=as_prog(pa, a, pra, M), pro_b=as_prog(pb, bt, prb, N))
+            elif Kx % 8 == 0 and K.contract_any(a, (*pa.strides, 1), bt, (*pb.strides, 1), (B, M, N, Kx), prog,
+                                                [vals[i] for i in eslots], out):
+                pass  # k split over workgroups where the grid is small
             elif KP == Kx:  # every operand as stored (or as packed), through its strides
                 K.contract_strided(a, pa.strides, bt, pb.strides, (B, M, N, Kx), prog,
                                    [vals[i] for i in eslots], out, f32_mode=self.f32_contract)

@@ -732,6 +732,43 @@ def _contraction_runner(region, cb, grid, dtype):
 
     fused = dtype in ("f32", "bf16") and "chain" in (pa[0], pb[0])
     bound: list = []  # the epilogue program
+    in_place = None  # the params' (batch, row, k) strides, where the kernel reads them as they are stored
+    if not fused and pa[0] == pb[0] == "param":
+
+        def strides(node, row):
+            st = dict(zip(node.type.names, _dense(node.type.shape)))
+            sk = st[k]
+            # a single row takes any stride
+            return (st.get(lnames[0], 0), st[row] if row in st else (KP if sk == 1 else 1), sk)
+
+        in_place = (strides(cb["a"], lnames[1]), strides(cb["b"], lnames[2]))
+        if dtype == "f32":
+            if any(sk != 1 and sr != 1 for _sb, sr, sk in in_place):
+                in_place = None
+        elif not (K.any_layout(Kdim, M_, *in_place[0]) and K.any_layout(Kdim, N_, *in_place[1])):
+            in_place = None
+    split: list = []  # fp32: k slices, the partial sums' program and the finish, made by the first call
+
+    def contract_in_place(torch, a, bt, prog, ops, out):
+        """Whether the contraction ran on the params where they lie: 16-bit
+        through pdh_contract_any, fp32 through pdh_contract_views (its k in
+        slices where the output's tiles cannot fill the chip, as the carved-plan
+        executor picks them)."""
+        (sta, stb), shape4 = in_place, (B_, M_, N_, Kdim)
+        if dtype != "f32":
+            return K.contract_any(a, sta, bt, stb, shape4, prog, ops, out)
+        if not split:
+            split.append(ewprog.pick_ksplit(prog, B_, M_, N_, KP // 64))
+        S, ident, fin = split[0]
+        if S == 1:
+            K.contract_views(a, sta, bt, stb, shape4, prog, ops, out)
+            return True
+        ws = torch.empty((B_ * S, M_, N_), device="cuda", dtype=torch.float32)
+        K.contract_views(a, sta, bt, stb, shape4, ident, [], ws, ksplit=S)
+        p0, plane = ws.data_ptr(), 4 * M_ * N_
+        K.map_chain_bound(fin, [p0 + s * plane for s in range(S)] + [t.data_ptr() for t in ops], out)
+        return True
+
     present = [nm for nm in lnames if nm in y.type.names]  # the unit stand-ins drop out
     full_shape = tuple(size[nm].size for nm in present)
     full_perm = [present.index(nm) for nm in y.type.names]
@@ -778,7 +815,7 @@ def _contraction_runner(region, cb, grid, dtype):
                     sides.append((t, t.stride(), None))
             (a, sta, pra), (bt, stb, prb) = sides
             K.contract_views_pro(a, sta, bt, stb, (B_, M_, N_, Kdim), prog, ops, out, pro_a=pra, pro_b=prb)
-        else:
+        elif in_place is None or not contract_in_place(torch, ts[pa[1]], ts[pb[1]], prog, ops, out):
             a = build(pa, cb["a"], a_order, M_)
             bt = build(pb, cb["b"], b_order, N_)
             K.contract(a, bt, Kdim, prog, ops, out)

@@ -10,6 +10,7 @@ fusion.py:517-523, with batch and head as independent instances)."""
 from __future__ import annotations
 
 import ctypes as C
+import functools
 import math
 from dataclasses import dataclass
 
@@ -597,6 +598,55 @@ def contract_views(a: torch.Tensor, a_strides, bt: torch.Tensor, bt_strides, sha
         "pdh_contract_views", _ptr(a), *sa, _ptr(bt), *sb_, B, M, N, Kd, int(ksplit), C.byref(epi), table,
         _ptr(out), _DT[a.dtype], _stream()))
     return out
+
+
+def any_layout(k: int, rows: int, sb: int, sr: int, sk: int) -> bool:
+    """Whether :func:`contract_any` reads an operand of ``rows`` rows at these
+    (batch, row, k) element strides: 16-byte chunks along k, or along the rows."""
+    if k % 8 or sb % 8 or min(sb, sr, sk) < 0:
+        return False
+    return (sk == 1 and sr >= k and sr % 8 == 0) or (sr == 1 and sk >= rows and sk % 8 == 0 and rows % 8 == 0)
+
+
+def contract_any(a: torch.Tensor, a_strides, bt: torch.Tensor, bt_strides, shape, epi: _lib.EwProgram,
+                 operands: list, out: torch.Tensor) -> bool:
+    """The 16-bit contraction over operands read in place (pdh_contract_any):
+    acc[b, m, n] = sum_k a[b, m, k] bt[b, n, k], a[b, m, k] at element
+    b sa_b + m sa_r + k sa_k of ``a`` (``a_strides`` = (sa_b, sa_r, sa_k)), each
+    operand with k or its rows contiguous (:func:`any_layout`); ``shape`` =
+    (batch, m, n, k). False (nothing launched) where the operands do not lie
+    that way or the specialized kernels are off: the caller packs them."""
+    B, M, N, Kd = shape
+    if a.dtype not in (torch.bfloat16, torch.float16) or bt.dtype != a.dtype or out.dtype != a.dtype:
+        return False
+    if not any_layout(Kd, M, *a_strides) or not any_layout(Kd, N, *bt_strides):
+        return False
+    _require_cuda(a, bt, out, *operands)
+    pa, pb = a.data_ptr(), bt.data_ptr()
+    if (pa | pb) & 15:
+        return False
+    for t, (sb, sr, sk), rows in ((a, a_strides, M), (bt, bt_strides, N)):
+        reach = t.storage_offset() + (B - 1) * sb + (rows - 1) * sr + (Kd - 1) * sk + 1
+        if reach > t.untyped_storage().nbytes() // t.element_size():
+            raise ValueError("a strided operand's view reaches past its storage")
+    if epi.ndim != 3 or tuple(epi.shape[d] for d in range(3)) != (B, M, N):
+        raise ValueError("the epilogue's lattice must be (batch, m, n)")
+    _check_views(epi, operands, out, 3)
+    need = _any_workspace(B, M, N, Kd)
+    ws = out.new_empty(need // 4, dtype=torch.float32) if need else None
+    table = (C.c_void_p * max(1, len(operands)))(*[t.data_ptr() for t in operands])
+    code = _lib.lib().pdh_contract_any(
+        pa, *a_strides, pb, *bt_strides, B, M, N, Kd, C.byref(epi), table, out.data_ptr(), _DT[a.dtype], _ptr(ws), need,
+        _stream())
+    if code == _lib.PDH_EUNSUPPORTED:
+        return False
+    _lib.check("pdh_contract_any", code)
+    return True
+
+
+@functools.lru_cache(maxsize=4096)
+def _any_workspace(batch: int, m: int, n: int, k: int) -> int:
+    return _lib.lib().pdh_contract_any_workspace(batch, m, n, k)
 
 
 def contract_views_pro(a, a_strides, bt, bt_strides, shape, epi: _lib.EwProgram, operands: list,
