@@ -27,7 +27,7 @@
 // -> 163 us and forward 182 -> 58 us; 32 heads x 2048, D = 64, all keys live:
 // forward 119 TFLOP/s, backward 109 (seven products, the dQ role recomputes
 // two) of the 157 the fp32 matrix cores peak at; one head x 256: 29 -> 7.3 us.
-// The distance to 64 bits is the VALU kernels' or smaller (o 2.8e-7, dK 8e-7 of
+// The distance to 64 bits is the VALU kernels' or smaller (o 1.8e-7, dK 8e-7 of
 // the norm at 24 x 1000).
 #include "attn_f32.h"
 
@@ -205,9 +205,14 @@ __global__ __launch_bounds__(64 * WQ * WK, 2) void attn_f32_fwd(AttnF32Args a) {
     }
     const unsigned char* kt_ = smem + buf * 2 * T::BYTES + 16 * KH * wk * T::ROWB;
     const unsigned char* vt_ = kt_ + T::BYTES;
-    f32x4 s[KH];
+    // Short chains of sums, as a wave's lanes had before the matrix cores: the
+    // even and the odd chunks of D apart, and each step's P V added to o as a
+    // whole. One chain over D and one over the keys was 1-4% faster but left o
+    // 2.81e-7 from 64 bits at 24 heads x 1000 causal and 5.1e-7 at 64 heads x
+    // 270 x 1232, D = 64 (the VALU kernel: 2.56e-7, 4.2e-7); these: 1.76e-7, 2.3e-7.
+    f32x4 s[KH], s1[KH];
 #pragma unroll
-    for (int h = 0; h < KH; ++h) s[h] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int h = 0; h < KH; ++h) s[h] = s1[h] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int x = 0; x < NS; ++x) {
       f32x4 kf[KH];
@@ -216,11 +221,14 @@ __global__ __launch_bounds__(64 * WQ * WK, 2) void attn_f32_fwd(AttnF32Args a) {
 #pragma unroll
       for (int j = 0; j < 4; ++j)
 #pragma unroll
-        for (int h = 0; h < KH; ++h) s[h] = mfma4(kf[h][j], q[x][j], s[h]);
+        for (int h = 0; h < KH; ++h) {
+          f32x4& t = x & 1 ? s1[h] : s[h];
+          t = mfma4(kf[h][j], q[x][j], t);
+        }
     }
     float mx = m;
 #pragma unroll
-    for (int h = 0; h < KH; ++h) s[h] *= a.scale;
+    for (int h = 0; h < KH; ++h) s[h] = (s[h] + s1[h]) * a.scale;
     if (cut) {
 #pragma unroll
       for (int h = 0; h < KH; ++h)
@@ -248,16 +256,22 @@ __global__ __launch_bounds__(64 * WQ * WK, 2) void attn_f32_fwd(AttnF32Args a) {
       }
     l = l * alpha + ps;
     m = mx;
-    if (__any(alpha != 1.0f)) {
 #pragma unroll
-      for (int f = 0; f < NS; ++f) o[f] *= alpha;
+    for (int f0 = 0; f0 < NS; f0 += 4) {
+      f32x4 pv[4];
+#pragma unroll
+      for (int f = 0; f < 4; ++f) pv[f] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int h = 0; h < KH; ++h)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+          for (int f = 0; f < 4; ++f) pv[f] = mfma4(off.feature(vt_, h, f0 + f, j), s[h][j], pv[f]);
+#pragma unroll
+      for (int f = 0; f < 4; ++f)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) o[f0 + f][i] = __builtin_fmaf(o[f0 + f][i], alpha, pv[f][i]);
     }
-#pragma unroll
-    for (int h = 0; h < KH; ++h)
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-#pragma unroll
-        for (int f = 0; f < NS; ++f) o[f] = mfma4(off.feature(vt_, h, f, j), s[h][j], o[f]);
   };
   auto step = [&](int kt, auto bufc) __attribute__((always_inline)) {
     wait_vmcnt0();
