@@ -5,7 +5,8 @@
 // MFMA kernel (bf16 / f16 in, fp32 accumulate), e == od == D in {64, 128}:
 //   * workgroup = 4 waves x 32 query rows = 128 rows; key tiles of 32 rows,
 //     double-buffered in LDS (32 KB at D = 128): three workgroups share a CU,
-//     so three waves per SIMD overlap each other's LDS / MFMA / VALU latency;
+//     so three waves per SIMD overlap each other's LDS / MFMA / VALU latency
+//     (small or uneven grids take other workgroups: launch_mfma);
 //   * K and V tiles go HBM -> LDS by direct buffer loads (no VGPR staging, no
 //     LDS write instructions) into unpadded rows whose 16-byte slots are
 //     XOR-swizzled so every operand read is bank-conflict free;
@@ -194,17 +195,22 @@ __device__ __forceinline__ BlockPlan block_plan(const FwdArgs& a) {
 // rows). So, as in the 32x32x16 kernel, the score accumulators feed the
 // second product with no register shuffle.
 
-template <int D>
+// WQ x WK waves: wave (wq, wk) owns query rows 32 wq .. of the workgroup's
+// 32 WQ and the key tiles of index wk mod WK, staged by its group's WQ waves.
+template <int D, int WQ = 4, int WK = 1>
 struct F16Cfg {
-  static constexpr int WAVES = 4;
-  static constexpr int THREADS = 64 * WAVES;
-  static constexpr int BM = 32 * WAVES;    // query rows per workgroup (32 per wave)
+  static constexpr int WAVES = WQ;         // waves that stage a tile
+  static constexpr int THREADS = 64 * WQ * WK;
+  static constexpr int BM = 32 * WQ;       // query rows per workgroup (32 per wave)
   static constexpr int BN = 32;            // keys per tile
   static constexpr int ROWB = D * 2;       // LDS bytes per key row (swizzled, unpadded)
   static constexpr int CPR = D / 8;        // 16-byte chunks per row
   static constexpr int TILEB = BN * ROWB;  // one K or V tile
   static constexpr int KBUF = 0, VBUF = 2 * TILEB;
-  static constexpr int LDS = 4 * TILEB;    // K and V, double buffered: 32 KB at D = 128
+  static constexpr int GROUPB = 4 * TILEB; // a key group's K and V, double buffered: 32 KB at D = 128
+  // the key groups' states, merged at the end: one 16-row half of o per wave at a time, and (m, true m, l)
+  static constexpr int STATEB = (WK - 1) * WQ * 64 * (D / 16 * 16 + 6 * 4);
+  static constexpr int LDS = WK * GROUPB > STATEB ? WK * GROUPB : STATEB;
   static constexpr int RPK = 1024 / ROWB;  // rows per 1 KB direct-load block
   static constexpr int NBLK = TILEB / 1024;
   static constexpr int NDMA = (NBLK + WAVES - 1) / WAVES;
@@ -295,11 +301,13 @@ __device__ __forceinline__ void fwd16_store(const FwdArgs& a, int64_t inst, int 
   }
 }
 
-template <typename T, int D, bool ART>
-__global__ __launch_bounds__(F16Cfg<D>::THREADS, 3) void flash_fwd_m16(FwdArgs a) {
-  using C = F16Cfg<D>;
+template <typename T, int D, bool ART, int WQ = 4, int WK = 1>
+__global__ __launch_bounds__(64 * WQ * WK, WK > 1 ? 2 : 3) void flash_fwd_m16(FwdArgs a) {
+  using C = F16Cfg<D, WQ, WK>;
   __shared__ __attribute__((aligned(1024))) unsigned char smem[C::LDS];
-  const int tid = threadIdx.x, lane = tid & 63, w = wave_id(), c = lane & 15, G = lane >> 4;
+  const int lane = threadIdx.x & 63, c = lane & 15, G = lane >> 4;
+  const int w = WK == 1 ? wave_id() : wave_id() % WQ, wk = WK == 1 ? 0 : wave_id() / WQ;  // row group, key group
+  unsigned char* const gsm = smem + (WK == 1 ? 0 : wk * C::GROUPB);                       // the key group's tiles
 
   const BlockPlan bp = block_plan<C::BM, C::BN>(a);
   const int64_t inst = bp.inst;
@@ -346,8 +354,8 @@ __global__ __launch_bounds__(F16Cfg<D>::THREADS, 3) void flash_fwd_m16(FwdArgs a
       const int blk = i * C::WAVES + w;
       if (C::NBLK % C::WAVES != 0 && blk >= C::NBLK) break;
       const uint32_t row0 = static_cast<uint32_t>(tile * C::BN + blk * C::RPK);
-      dma16(kr, smem + C::KBUF + buf * C::TILEB + blk * 1024, dk[i], row0 * grk);
-      dma16(vr, smem + C::VBUF + buf * C::TILEB + blk * 1024, dv[i], row0 * grv);
+      dma16(kr, gsm + C::KBUF + buf * C::TILEB + blk * 1024, dk[i], row0 * grk);
+      dma16(vr, gsm + C::VBUF + buf * C::TILEB + blk * 1024, dv[i], row0 * grv);
     }
   };
 
@@ -377,8 +385,8 @@ __global__ __launch_bounds__(F16Cfg<D>::THREADS, 3) void flash_fwd_m16(FwdArgs a
   auto tile = [&](auto bufc, int key0, auto cutc) {
     constexpr bool CUT = decltype(cutc)::value;
     constexpr int buf = decltype(bufc)::value;
-    const unsigned char* kt = smem + C::KBUF + buf * C::TILEB;
-    const unsigned char* vt = smem + C::VBUF + buf * C::TILEB;
+    const unsigned char* kt = gsm + C::KBUF + buf * C::TILEB;
+    const unsigned char* vt = gsm + C::VBUF + buf * C::TILEB;
     f32x4 sacc[2][2];  // [key half][query half]: S^T[16 kb + 4 G + i][16 h + c]
 #pragma unroll
     for (int kb = 0; kb < 2; ++kb) sacc[kb][0] = sacc[kb][1] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -485,35 +493,111 @@ __global__ __launch_bounds__(F16Cfg<D>::THREADS, 3) void flash_fwd_m16(FwdArgs a
     __builtin_amdgcn_s_setprio(0);
   };
 
-  if (kt_lo < kt_hi) stage(kt_lo, 0);
-  auto one = [&](int kt, auto bufc, auto cutc) {
-    constexpr int buf = decltype(bufc)::value;
-    wait_vmcnt0();
-    __syncthreads();
-    if (kt + 1 < kt_hi) stage(kt + 1, buf ^ 1);
-    const int key0 = kt * C::BN;
-    bool dead = false;
-    if (decltype(cutc)::value && a.masked && a.prune) {  // this wave's rows see no live key here
-      const int dmin = key0 - (qw0 + 31), dmax = key0 + C::BN - 1 - qw0;
-      dead = dmin > a.band_hi32 || dmax < a.band_lo32;
+  if constexpr (WK == 1) {
+    if (kt_lo < kt_hi) stage(kt_lo, 0);
+    auto one = [&](int kt, auto bufc, auto cutc) {
+      constexpr int buf = decltype(bufc)::value;
+      wait_vmcnt0();
+      __syncthreads();
+      if (kt + 1 < kt_hi) stage(kt + 1, buf ^ 1);
+      const int key0 = kt * C::BN;
+      bool dead = false;
+      if (decltype(cutc)::value && a.masked && a.prune) {  // this wave's rows see no live key here
+        const int dmin = key0 - (qw0 + 31), dmax = key0 + C::BN - 1 - qw0;
+        dead = dmin > a.band_hi32 || dmax < a.band_lo32;
+      }
+      if (!dead) tile(bufc, key0, cutc);
+    };
+    auto sweep = [&](int from, int to, auto cutc) {
+      int kt = from;
+      if (kt < to && ((kt - kt_lo) & 1)) one(kt++, std::integral_constant<int, 1>{}, cutc);
+      for (; kt + 1 < to; kt += 2) {
+        one(kt, std::integral_constant<int, 0>{}, cutc);
+        one(kt + 1, std::integral_constant<int, 1>{}, cutc);
+      }
+      if (kt < to) one(kt, std::integral_constant<int, 0>{}, cutc);
+    };
+    sweep(kt_lo, kf_lo, std::true_type{});
+    sweep(kf_lo, kf_hi, std::false_type{});
+    sweep(kf_hi, kt_hi, std::true_type{});
+  } else {
+    // key group wk takes the tiles kt = wk (mod WK) of the absolute grid, one
+    // per step; every wave steps, so the barriers are the workgroup's
+    const int first = kt_lo - kt_lo % WK + wk;
+    const int steps = kt_lo < kt_hi ? (kt_hi - (kt_lo - kt_lo % WK) + WK - 1) / WK : 0;
+    auto live = [&](int kt) { return kt >= kt_lo && kt < kt_hi; };
+    auto one = [&](int i, auto bufc) __attribute__((always_inline)) {
+      constexpr int buf = decltype(bufc)::value;
+      const int kt = first + WK * i;
+      wait_vmcnt0();
+      __syncthreads();
+      if (i + 1 < steps && live(kt + WK)) stage(kt + WK, buf ^ 1);
+      if (!live(kt)) return;
+      const int key0 = kt * C::BN;
+      if (kt >= kf_lo && kt < kf_hi) {
+        tile(bufc, key0, std::false_type{});
+        return;
+      }
+      if (a.masked && a.prune) {  // this wave's rows see no live key here
+        const int dmin = key0 - (qw0 + 31), dmax = key0 + C::BN - 1 - qw0;
+        if (dmin > a.band_hi32 || dmax < a.band_lo32) return;
+      }
+      tile(bufc, key0, std::true_type{});
+    };
+    if (steps > 0 && live(first)) stage(first, 0);
+    for (int i = 0; i < steps; i += 2) {
+      one(i, std::integral_constant<int, 0>{});
+      if (i + 1 < steps) one(i + 1, std::integral_constant<int, 1>{});
     }
-    if (!dead) tile(bufc, key0, cutc);
-  };
-  auto sweep = [&](int from, int to, auto cutc) {
-    int kt = from;
-    if (kt < to && ((kt - kt_lo) & 1)) one(kt++, std::integral_constant<int, 1>{}, cutc);
-    for (; kt + 1 < to; kt += 2) {
-      one(kt, std::integral_constant<int, 0>{}, cutc);
-      one(kt + 1, std::integral_constant<int, 1>{}, cutc);
-    }
-    if (kt < to) one(kt, std::integral_constant<int, 0>{}, cutc);
-  };
-  sweep(kt_lo, kf_lo, std::true_type{});
-  sweep(kf_lo, kf_hi, std::false_type{});
-  sweep(kf_hi, kt_hi, std::true_type{});
+  }
   wait_vmcnt0();  // no load may be in flight into LDS when the workgroup exits
 
-  const float mt[2] = {ART ? mtrue[0] : mused[0], ART ? mtrue[1] : mused[1]};
+  float mt[2] = {ART ? mtrue[0] : mused[0], ART ? mtrue[1] : mused[1]};
+  if constexpr (WK > 1) {  // merge the key groups' states through LDS: the tiles are done with
+    constexpr int OB = C::FB * 64 * 16;  // bytes of one wave's half of o
+    float* const st = reinterpret_cast<float*>(smem + (WK - 1) * WQ * OB);
+    __syncthreads();
+    if (wk > 0) {
+      float* p = st + ((wk - 1) * WQ + w) * 6 * 64 + lane;
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        p[(3 * h) * 64] = mused[h];
+        p[(3 * h + 1) * 64] = mt[h];
+        p[(3 * h + 2) * 64] = lsum[h];
+      }
+    }
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      if (wk > 0) {
+        unsigned char* p = smem + ((wk - 1) * WQ + w) * OB + lane * 16;
+#pragma unroll
+        for (int fb = 0; fb < C::FB; ++fb) *reinterpret_cast<f32x4*>(p + fb * 1024) = oacc[fb][h];
+      }
+      __syncthreads();
+      if (wk == 0) {
+        float M = mused[h];
+#pragma unroll
+        for (int i = 0; i < WK - 1; ++i) M = fmaxf(M, st[((i * WQ + w) * 6 + 3 * h) * 64 + lane]);
+        const float w0 = mused[h] > -kInf ? fast_exp2((mused[h] - M) * a.c2) : 0.f;
+        lsum[h] *= w0;
+#pragma unroll
+        for (int fb = 0; fb < C::FB; ++fb) oacc[fb][h] *= w0;
+#pragma unroll
+        for (int i = 0; i < WK - 1; ++i) {
+          const float* p = st + ((i * WQ + w) * 6 + 3 * h) * 64 + lane;
+          const float wi = p[0] > -kInf ? fast_exp2((p[0] - M) * a.c2) : 0.f;  // a group without live keys adds nothing
+          mt[h] = fmaxf(mt[h], p[64]);
+          lsum[h] += p[128] * wi;
+          const unsigned char* po = smem + (i * WQ + w) * OB + lane * 16;
+#pragma unroll
+          for (int fb = 0; fb < C::FB; ++fb) oacc[fb][h] += *reinterpret_cast<const f32x4*>(po + fb * 1024) * wi;
+        }
+        mused[h] = M;
+      }
+      __syncthreads();  // before the other half takes the room
+    }
+    if (wk != 0) return;
+  }
   fwd16_store<T, D>(a, inst, bp.split, qw0, c, G, op, oacc, mused, mt, lsum);
 }
 
@@ -842,27 +926,28 @@ bool band_has_empty_row(int64_t T, int64_t S, int64_t lo, int64_t hi) {
 }
 
 
-template <typename T, int D>
+template <typename T, int D, int WQ = 4, int WK = 1>
 void fwd_kernel(const FwdArgs& a, unsigned nblocks, hipStream_t st) {
   if (a.m_out || a.den_out)
-    flash_fwd_m16<T, D, true><<<dim3(nblocks), F16Cfg<D>::THREADS, 0, st>>>(a);
+    flash_fwd_m16<T, D, true, WQ, WK><<<dim3(nblocks), 64 * WQ * WK, 0, st>>>(a);
   else
-    flash_fwd_m16<T, D, false><<<dim3(nblocks), F16Cfg<D>::THREADS, 0, st>>>(a);
+    flash_fwd_m16<T, D, false, WQ, WK><<<dim3(nblocks), 64 * WQ * WK, 0, st>>>(a);
 }
 
-template <typename T, int D>
-int launch_mfma(const FwdArgs& a, int64_t ninst, hipStream_t st) {
-  using C = F16Cfg<D>;
+template <typename T, int D, int WQ, int WK>
+int launch_as(const FwdArgs& a, int64_t ninst, hipStream_t st) {
+  using C = F16Cfg<D, WQ, WK>;
   static_assert(C::LDS <= 64 * 1024, "the forward's static LDS fits one workgroup's limit");
-  const int64_t nblk = ninst * a.nqb;
-  PDH_REQUIRE(nblk <= INT32_MAX, PDH_EINVAL, "pdh_flash_fwd: grid too large (%lld workgroups)", (long long)nblk);
   FwdArgs aa = a;
+  aa.nqb = static_cast<int>((a.t + C::BM - 1) / C::BM);
+  const int64_t nblk = ninst * aa.nqb;
+  PDH_REQUIRE(nblk <= INT32_MAX, PDH_EINVAL, "pdh_flash_fwd: grid too large (%lld workgroups)", (long long)nblk);
   if (a.nsplit > 1) {
     const int64_t ntiles = (a.s + C::BN - 1) / C::BN;
     aa.split_tiles = static_cast<int>((ntiles + a.nsplit - 1) / a.nsplit);
     aa.xcd_remap = 0;
     PDH_REQUIRE(nblk * a.nsplit <= INT32_MAX, PDH_EINVAL, "pdh_flash_fwd_split: grid too large");
-    fwd_kernel<T, D>(aa, static_cast<unsigned>(nblk * a.nsplit), st);
+    fwd_kernel<T, D, WQ, WK>(aa, static_cast<unsigned>(nblk * a.nsplit), st);
     int rc = check_launch("pdh_flash_fwd_split");
     if (rc) return rc;
     const int64_t nthr = a.plane * (D / 4);
@@ -870,9 +955,55 @@ int launch_mfma(const FwdArgs& a, int64_t ninst, hipStream_t st) {
     flash_fwd_combine<T, D><<<dim3(static_cast<unsigned>((nthr + 255) / 256)), 256, 0, st>>>(aa);
     return check_launch("pdh_flash_fwd_split (combine)");
   }
-  aa.xcd_remap = (nblk % 32 == 0 && a.nqb % 8 == 0) ? 3 : ((nblk % 8 == 0) ? 1 : 0);
-  fwd_kernel<T, D>(aa, static_cast<unsigned>(nblk), st);
+  aa.xcd_remap = (nblk % 32 == 0 && aa.nqb % 8 == 0) ? 3 : ((nblk % 8 == 0) ? 1 : 0);
+  fwd_kernel<T, D, WQ, WK>(aa, static_cast<unsigned>(nblk), st);
   return check_launch("pdh_flash_fwd");
+}
+
+// The workgroup of an unsplit sweep. Four waves of 32 query rows are the best
+// use of the staged keys, where their blocks fill the chip evenly; a grid of
+// fewer blocks than compute units, or a causal one whose blocks all start at
+// once (the longest then runs on alone), does better with 64-row blocks whose
+// waves share the keys and merge their states through LDS. Against splitting
+// the keys over workgroups this saves the partial states' round trip through
+// memory and the combine's launch. us, one launch (128-row blocks of four
+// waves; the split pick_fwd_splits takes), bf16, c = causal:
+//   heads x t x s x d       (4, 1)  split        here
+//   12 x 1024 c x 64         18.5    20.4   12.7 (2, 4)   [(2, 2) 13.8]
+//   16 x 2048 c x 64         31.4    30.3   26.6 (2, 2)   [(2, 4) 24.8]
+//   32 x 512 x 2048 x 64     29.0    26.9   18.1 (2, 4)   [(2, 2) 21.7]
+//   24 x 1024 x 2048 x 64    29.5    29.3   26.0 (2, 2)   [(2, 4) 32.2]
+//   32 x 512 c x 128         18.3    23.2   13.2 (2, 2)
+//   64 x 500 x 3001 x 128    73.5    80.4   61.3 (4, 2)   [(2, 2) 62.4]
+//   38 x 1024 c x 128        39.9    47.1   32.4 (2, 2)
+//   32 x 4096 c x 64        126.2      -    93.7 (2, 2)
+//   64 x 2048 c x 64         72.2      -    63.5 (2, 2);  x 128: 106.6, 107.2 kept
+// and past the lines: 64 x 1024 c x 64: 26.1 (4, 1), 28.0 (2, 2); 50 x 1024 x
+// 1024 x 64: 24.8, 29.6; 128 x 2048 c x 64: 100.2, 109.8; 53 keys: 5.4, 6.7.
+template <typename T, int D>
+int launch_mfma(const FwdArgs& a, int64_t ninst, hipStream_t st) {
+  if (a.nsplit == 1) {
+    static const int cus = pdh_device_cus() > 0 ? pdh_device_cus() : 256;
+    const int64_t blocks = ninst * a.nqb;  // of 128 rows
+    const bool lo = a.masked && a.band_lo > INT64_MIN / 4, hi = a.masked && a.band_hi < INT64_MAX / 4;
+    int64_t keys = a.s;  // a row's live keys, at most
+    if (lo && hi) {
+      const int64_t width = static_cast<int64_t>(a.band_hi32) - a.band_lo32 + 128;
+      keys = width < keys ? width : keys;
+    }
+    const bool uneven = lo != hi;  // the blocks' sweeps differ in length
+    if (blocks <= cus && keys >= 256) {
+      if constexpr (D == 64) {
+        if (2 * blocks <= cus && keys >= 1024) return launch_as<T, D, 2, 4>(a, ninst, st);
+      } else {
+        if (2 * blocks > cus && !uneven) return launch_as<T, D, 4, 2>(a, ninst, st);
+      }
+      return launch_as<T, D, 2, 2>(a, ninst, st);
+    }
+    if (uneven && ((2 * blocks <= 3 * cus && keys >= 512) || (blocks <= (D == 64 ? 4 : 2) * cus && keys >= 2048)))
+      return launch_as<T, D, 2, 2>(a, ninst, st);
+  }
+  return launch_as<T, D, 4, 1>(a, ninst, st);
 }
 
 }  // namespace

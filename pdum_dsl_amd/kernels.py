@@ -265,11 +265,11 @@ def flash_fwd(
     Returns the output plus lse and, with ``want_artifacts``, the reference's
     (m, den) artifacts ([B, H, T] fp32). ``nsplit`` > 1 splits each query
     block's keys over that many workgroups (pdh_flash_fwd_split); None picks
-    it (``pick_fwd_splits``): 1 unless the grid is too small to fill the chip."""
+    it (``_fwd_splits``): 1 unless the grid is small and its rows are long."""
     _require_cuda(q, k, v)
     if not (q.dtype == k.dtype == v.dtype) or q.dtype not in _DT:
         raise ValueError(f"q/k/v must share one dtype of f32/bf16/f16 (got {q.dtype}, {k.dtype}, {v.dtype})")
-    B, H, T, _ = q.shape
+    B, H, T, E = q.shape
     o = q.new_empty((B, H, T, v.shape[3])) if out is None else out
     g = _geom(q, k, v, o)
     lse = q.new_empty((B, H, T), dtype=torch.float32) if want_lse else None
@@ -278,7 +278,7 @@ def flash_fwd(
     sc = 1.0 / math.sqrt(q.shape[3]) if scale is None else float(scale)
     kind, (lo, hi) = (PDH_MASK_NONE, (0, 0)) if band is None else (PDH_MASK_BAND, band.c_args())
     if nsplit is None:
-        nsplit = pick_fwd_splits(B * H, T, k.shape[2]) if q.dtype != torch.float32 else 1
+        nsplit = _fwd_splits(B * H, T, k.shape[2], E, band) if q.dtype != torch.float32 else 1
     if nsplit > 1 and q.dtype != torch.float32:
         need = _lib.lib().pdh_flash_fwd_workspace(C.byref(g), int(nsplit))
         ws = torch.empty((need + 3) // 4, dtype=torch.float32, device=q.device)
@@ -351,6 +351,27 @@ def pick_fwd_splits(ninst: int, t: int, s: int, cus: int | None = None) -> int:
     if blocks == 0 or blocks >= 2 * cus or ntiles < 16:
         return 1
     return int(max(1, min(ntiles // 8, (3 * cus) // blocks, 64)))
+
+
+def _fwd_splits(ninst: int, t: int, s: int, d: int, band: Band | None, cus: int | None = None) -> int:
+    """Key splits of a forward that names none: 1 where one launch whose waves
+    share the keys inside a workgroup (launch_mfma in flash_fwd.hip) measured
+    faster than ``pick_fwd_splits``' workgroups and their combine. It is slower
+    only where few blocks have long rows (bf16, us, one launch / split: 12 heads
+    x 1024 x 8192 keys 51 / 44 at d = 64, 104 / 75 at 128; one causal head x
+    4096 54 / 37 at 128; 8 heads x 1024 x 4096 29 / 30 at 64; 16 heads x 1024 x
+    4096 55 / 60 at 128) and in even grids of 1 to 2 blocks a compute unit."""
+    if cus is None:
+        cus = _cus()
+    blocks = ninst * ((t + 127) // 128)
+    lo, hi = (None, None) if band is None else (band.lo, band.hi)
+    keys = s if lo is None or hi is None else min(s, hi - lo + 128)
+    if blocks <= cus and keys >= 256 and not (keys >= 8192 and 2 * blocks <= cus) and not (
+            d == 128 and keys >= 4096 and 4 * blocks <= cus):
+        return 1
+    if blocks > cus and (lo is None) != (hi is None) and 2 * blocks <= 3 * cus and keys >= 512:
+        return 1
+    return pick_fwd_splits(ninst, t, s, cus)
 
 
 def flash_bwd(

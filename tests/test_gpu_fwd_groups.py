@@ -1,0 +1,93 @@
+"""The 16-bit forward whose waves share a block's keys and merge their states
+through LDS: every workgroup shape the launcher picks, at ragged rows and
+keys, bands and grouped heads, against float64; pruned and unpruned sweeps bit
+for bit; and which shapes still split their keys over workgroups (CPU)."""
+
+import pytest
+
+torch = pytest.importorskip("torch")
+
+
+def test_key_splits_only_for_few_blocks_with_long_rows():
+    from pdum_dsl_amd.kernels import Band, _fwd_splits, pick_fwd_splits
+
+    causal, window = Band(None, 0), Band(-255, 0)
+    for (n, t, s, d, band), want in {
+        (12, 1024, 1024, 64, causal): 1,
+        (64, 500, 3001, 128, None): 1,
+        (38, 1024, 1024, 128, causal): 1,
+        (12, 1024, 8192, 64, window): 1,  # under 384 live keys a row
+    }.items():
+        assert _fwd_splits(n, t, s, d, band, cus=256) == want
+    for n, t, s, d, band in ((12, 1024, 8192, 64, None), (1, 4096, 4096, 128, causal), (38, 1024, 4096, 128, None),
+                             (4, 255, 255, 64, None), (1, 1, 1, 64, None)):
+        assert _fwd_splits(n, t, s, d, band, cus=256) == pick_fwd_splits(n, t, s, cus=256)
+
+
+def _exact(q, k, v, band, fill, scale):
+    """(o, sum p |v|, largest sum |q| |k|, lse) in float64."""
+    q, k, v = (x.double().cpu() for x in (q, k, v))
+    r = q.shape[1] // k.shape[1]
+    k, v = (x.repeat_interleave(r, 1) for x in (k, v))
+    s = torch.matmul(q, k.transpose(2, 3)) * scale
+    size = float((torch.matmul(q.abs(), k.abs().transpose(2, 3)) * scale).max())
+    if band is not None:
+        d = torch.arange(s.shape[3])[None] - torch.arange(s.shape[2])[:, None]
+        dead = torch.zeros_like(d, dtype=torch.bool)
+        if band.lo is not None:
+            dead |= d < band.lo
+        if band.hi is not None:
+            dead |= d > band.hi
+        s = s.masked_fill(dead, fill)
+    p = torch.softmax(s, -1)
+    return torch.matmul(p, v), torch.matmul(p, v.abs()), size, torch.logsumexp(s, -1)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dt", ["bfloat16", "float16"])
+@pytest.mark.parametrize(
+    "B,H,Hkv,T,S,D,band",
+    [
+        # four key groups, 64-row blocks
+        (1, 1, 1, 1, 1024, 64, None),
+        (1, 2, 1, 65, 1055, 64, (None, 990)),
+        (1, 3, 3, 1030, 1024, 64, (None, 0)),
+        # two key groups, 64-row blocks
+        (1, 2, 2, 63, 256, 64, None),
+        (1, 4, 1, 130, 321, 64, (None, 2)),
+        (2, 2, 1, 200, 1500, 64, (-300, 5)),  # a window: fewer live keys than stored
+        (1, 1, 1, 33, 257, 128, (None, -1)),  # a fully masked row: no prune
+        (1, 8, 2, 300, 417, 128, (None, 0)),
+        (1, 6, 6, 129, 300, 128, (120, None)),
+        # two key groups, 128-row blocks
+        (3, 24, 12, 190, 287, 128, None),
+        # uneven sweeps over more blocks than compute units
+        (2, 70, 70, 257, 515, 64, (None, 100)),
+        (1, 36, 36, 2048, 2048, 64, (None, 0)),
+        (1, 100, 50, 400, 513, 128, (None, 0)),
+    ],
+)
+def test_grouped_keys_match_float64(B, H, Hkv, T, S, D, band, dt):
+    from pdum_dsl_amd import kernels as K
+
+    dt = getattr(torch, dt)
+    g = torch.Generator(device="cuda").manual_seed(T + S + D)
+    q, k, v = (torch.randn(B, h, n, D, generator=g, device="cuda").to(dt) for h, n in ((H, T), (Hkv, S), (Hkv, S)))
+    bnd, scale = (None if band is None else K.Band(*band)), D**-0.5
+    got = K.flash_fwd(q, k, v, band=bnd, nsplit=1)
+    full = K.flash_fwd(q, k, v, band=bnd, nsplit=1, prune=False)
+    arts = K.flash_fwd(q, k, v, band=bnd, nsplit=1, want_artifacts=True)
+    torch.cuda.synchronize()
+    assert torch.equal(got.o, full.o) and torch.equal(got.lse, full.lse)
+    want, mag, size, lse = _exact(q, k, v, bnd, -1e9, scale)
+    # p and o round to 16 bits (half an ulp each); a score is a sum of D fp32 products, and its error
+    # moves every p of the row (and the sum under it) by as much
+    unit = 2.0**-8 if dt == torch.bfloat16 else 2.0**-11
+    ds = (D + 16) * 2.0**-24 * size + 2.0**-20
+    bound = 1.01 * unit * (mag + want.abs()) + 3 * ds * mag + 2.0**-24
+    for out in (got, arts):
+        err = (out.o.double().cpu() - want).abs()
+        assert bool((err <= bound).all()), float((err / bound).max())
+        # lse of a fully masked row is the fill's own: compare relative to its size
+        assert bool(((out.lse.double().cpu() - lse).abs() <= 2 * ds + 2.0**-22 * lse.abs()).all())
+    assert bool(((arts.m + torch.log(arts.den) - arts.lse).abs() <= 1e-5 + 2.0**-21 * arts.lse.abs()).all())
