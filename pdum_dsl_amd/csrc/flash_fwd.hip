@@ -45,6 +45,8 @@
 #include "attn_common.h"
 #include "attn_f32.h"
 
+#include <cmath>
+#include <limits>
 #include <type_traits>
 
 namespace pdh {
@@ -284,7 +286,7 @@ __device__ __forceinline__ void fwd16_store(const FwdArgs& a, int64_t inst, int 
       }
       continue;
     }
-    const float inv = den > 0.f ? 1.0f / den : 0.f;
+    const float inv = 1.0f / den;  // den is 0 only where every score is -inf: NaN, as softmax has it
     uint16_t* obase = op + static_cast<int64_t>(qw0 + 16 * h) * a.o_st;  // wave-uniform
     const uint32_t o_lane = static_cast<uint32_t>(c * a.o_st * 2 + G * 8);
 #pragma unroll
@@ -431,16 +433,19 @@ __global__ __launch_bounds__(64 * WQ * WK, WK > 1 ? 2 : 3) void flash_fwd_m16(Fw
       }
     }
     u32x4 p[2];
-    // the tile's exponentials of query half h into p[h]; returns their sum
-    auto expo = [&](int h) {
-      const float mc = mused[h] * a.c2;
+    // What the exponentials refer to: a row's maximum, or 0 while all its
+    // scores are -inf (a fill of -inf), whose exponentials are then 0, not NaN.
+    auto ref = [&](int h) { return mused[h] == -kInf ? 0.f : mused[h]; };
+    // the tile's exponentials of query half h, referred to m, into p[h]; returns their sum
+    auto expo = [&](int h, float m) {
+      const float mc = m * a.c2;
       float e[8];
 #pragma unroll
       for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const float x = sacc[kb][h][i];
-          e[4 * kb + i] = CUT ? fast_exp2((x - mused[h]) * a.c2) : fast_exp2(__builtin_fmaf(x, a.c2, -mc));
+          e[4 * kb + i] = CUT ? fast_exp2((x - m) * a.c2) : fast_exp2(__builtin_fmaf(x, a.c2, -mc));
         }
       p[h] = u32x4{pack2<T>(e[0], e[1]), pack2<T>(e[2], e[3]), pack2<T>(e[4], e[5]), pack2<T>(e[6], e[7])};
       return ((e[0] + e[1]) + (e[2] + e[3])) + ((e[4] + e[5]) + (e[6] + e[7]));
@@ -461,13 +466,14 @@ __global__ __launch_bounds__(64 * WQ * WK, WK > 1 ? 2 : 3) void flash_fwd_m16(Fw
       for (int fb = 0; fb < C::FB; ++fb) oacc[fb][h] *= alpha;
     };
     if constexpr (!CUT && !ART) {
-      float part0 = expo(0), part1 = expo(1);
+      // a maximum still at -inf makes these inf or NaN: over the limit
+      float part0 = expo(0, mused[0]), part1 = expo(1, mused[1]);
       const float lim = static_cast<float>(1 << static_cast<int>(kTau));
       if (__builtin_amdgcn_ballot_w64(!(part0 <= lim) || !(part1 <= lim)) != 0) {
         rescale(0, fmaxf(mused[0], rowmax(0)));
         rescale(1, fmaxf(mused[1], rowmax(1)));
-        part0 = expo(0);
-        part1 = expo(1);
+        part0 = expo(0, ref(0));
+        part1 = expo(1, ref(1));
       }
       lsum[0] += part0;
       lsum[1] += part1;
@@ -479,8 +485,8 @@ __global__ __launch_bounds__(64 * WQ * WK, WK > 1 ? 2 : 3) void flash_fwd_m16(Fw
         rescale(0, fmaxf(mused[0], m0));
         rescale(1, fmaxf(mused[1], m1));
       }
-      lsum[0] += expo(0);
-      lsum[1] += expo(1);
+      lsum[0] += expo(0, ref(0));
+      lsum[1] += expo(1, ref(1));
     }
     __builtin_amdgcn_s_setprio(1);
 #pragma unroll
@@ -904,7 +910,7 @@ __global__ __launch_bounds__(256) void flash_fwd_combine(FwdArgs a) {
     const f32x4 oc = *reinterpret_cast<const f32x4*>(a.ws + (c * P + row) * D + 4 * f4);
     acc += oc * w;
   }
-  const float inv = den > 0.f ? 1.0f / den : 0.f;
+  const float inv = 1.0f / den;  // as fwd16_store
   const int64_t inst = row / a.t, tq = row % a.t;
   const int64_t b = inst / a.heads_q, hq = inst % a.heads_q;
   uint16_t* orow = static_cast<uint16_t*>(a.o) + b * a.o_sb + hq * a.o_sh + tq * a.o_st + 4 * f4;
@@ -1087,9 +1093,12 @@ int flash_fwd_impl(const void* q, const void* k, const void* v, void* o, float* 
               "pdh_flash_fwd: row strides must be < 2^24 elements");
   PDH_REQUIRE(G.s * G.k_st * 2 < INT32_MAX && G.s * G.v_st * 2 < INT32_MAX, PDH_EINVAL,
               "pdh_flash_fwd: one instance's K / V rows must span < 2 GiB");
+  // the masked raw score: a finite fill stays finite (the lowest fp32 value over a scale under 1 would not)
+  float fill_raw = fill / scale;
+  if (std::isinf(fill_raw) && !std::isinf(fill)) fill_raw = std::copysign(std::numeric_limits<float>::max(), fill);
   FwdArgs a{q, k, v, o, m_out, den_out, lse_out, G.heads_q, G.heads_kv, G.t, G.s,
             G.q_sb, G.q_sh, G.q_st, G.k_sb, G.k_sh, G.k_st, G.v_sb, G.v_sh, G.v_st, G.o_sb, G.o_sh, G.o_st,
-            scale, scale * kLog2e, fill / scale, masked, band_lo, band_hi, prune_ok,
+            scale, scale * kLog2e, fill_raw, masked, band_lo, band_hi, prune_ok,
             static_cast<int>((G.t + F16Cfg<128>::BM - 1) / F16Cfg<128>::BM), 0};
   {
     constexpr int64_t kBand32 = (int64_t{1} << 29) + 64;

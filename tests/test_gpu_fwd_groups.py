@@ -91,3 +91,55 @@ def test_grouped_keys_match_float64(B, H, Hkv, T, S, D, band, dt):
         # lse of a fully masked row is the fill's own: compare relative to its size
         assert bool(((out.lse.double().cpu() - lse).abs() <= 2 * ds + 2.0**-22 * lse.abs()).all())
     assert bool(((arts.m + torch.log(arts.den) - arts.lse).abs() <= 1e-5 + 2.0**-21 * arts.lse.abs()).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("fill", [float("-inf"), torch.finfo(torch.float32).min], ids=["-inf", "lowest"])
+@pytest.mark.parametrize(
+    "B,H,Hkv,T,S,D,band",
+    [
+        (1, 2, 1, 65, 1055, 64, (None, 990)),  # four key groups
+        (1, 4, 1, 130, 321, 64, (None, 2)),  # two: a group's first tile is dead for some of a wave's rows
+        (2, 2, 1, 200, 1500, 64, (-300, 5)),
+        (1, 1, 1, 33, 257, 128, (None, -1)),  # a fully masked row
+        (1, 6, 6, 129, 300, 128, (120, None)),
+        (3, 24, 12, 190, 287, 128, (None, 97)),
+        (2, 70, 70, 257, 230, 64, (-100, 2)),  # one key group
+        (2, 2, 1, 200, 90, 128, (-70, 3)),
+    ],
+)
+def test_the_lowest_fills_leave_live_rows_finite(B, H, Hkv, T, S, D, band, fill):
+    """A masked score of -inf, or of a finite fill that overflows over the
+    scale: a tile (or group, or split) in which a row sees nothing else adds
+    nothing to it. A row with no live key is NaN for -inf, the mean of V else."""
+    from pdum_dsl_amd import kernels as K
+
+    g = torch.Generator(device="cuda").manual_seed(T + S + D)
+    q, k, v = (torch.randn(B, h, n, D, generator=g, device="cuda").bfloat16() for h, n in ((H, T), (Hkv, S), (Hkv, S)))
+    bnd, scale = K.Band(*band), D**-0.5
+    kw = dict(band=bnd, fill=fill)
+    outs = [K.flash_fwd(q, k, v, nsplit=1, **kw), K.flash_fwd(q, k, v, nsplit=1, prune=False, **kw),
+            K.flash_fwd(q, k, v, nsplit=1, want_artifacts=True, **kw), K.flash_fwd(q, k, v, nsplit=3, **kw),
+            K.flash_fwd(q, k, v, nsplit=3, prune=False, want_artifacts=True, **kw)]
+    torch.cuda.synchronize()
+    want, mag, size, lse = _exact(q, k, v, bnd, fill, scale)
+    d = torch.arange(S)[None] - torch.arange(T)[:, None]
+    live = torch.ones_like(d, dtype=torch.bool)
+    if band[0] is not None:
+        live &= d >= band[0]
+    if band[1] is not None:
+        live &= d <= band[1]
+    live = live.any(1)  # rows with a live key
+    unit, ds = 2.0**-8, (D + 16) * 2.0**-24 * size + 2.0**-20  # as in test_grouped_keys_match_float64
+    bound = 1.01 * unit * (mag + want.abs()) + 3 * ds * mag + 2.0**-24
+    for out in outs:
+        o = out.o.double().cpu()
+        assert bool(((o - want).abs() <= bound)[:, :, live].all())
+        assert bool(((out.lse.double().cpu() - lse).abs() <= 2 * ds + 2.0**-22 * lse.abs())[:, :, live].all())
+        if fill == float("-inf"):
+            assert bool(torch.isnan(o[:, :, ~live]).all())
+        else:
+            assert bool(((o - want).abs() <= bound)[:, :, ~live].all())
+    assert torch.equal(outs[0].o[:, :, live.cuda()], outs[1].o[:, :, live.cuda()])
+    for art in (outs[2], outs[4]):
+        assert bool(((art.m + torch.log(art.den) - art.lse).abs() <= 1e-5 + 2.0**-21 * art.lse.abs())[:, :, live.cuda()].all())
