@@ -201,12 +201,80 @@ def _under_renames(n):
     return n
 
 
+@dataclass(frozen=True)
+class _GemmDims:
+    """The lattice of a GEMM-shaped contraction: one batch dim (or a unit
+    stand-in), the m and the n dims of its output (a unit dim where there are
+    none) and the contracted dims."""
+
+    kd: tuple  # contracted dim names
+    kdim: dict  # name -> Dim
+    riders: list
+    bdim: Dim
+    mdims: list
+    ndims: list
+    size: dict  # output dim name -> Dim
+
+    @property
+    def lattice(self) -> tuple:
+        return (self.bdim,) + tuple(self.size[nm] for nm in (*self.mdims, *self.ndims))
+
+
+def _gemm_dims(m) -> _GemmDims:
+    """The dims of a GEMM-shaped match (match_contraction_epilogue)."""
+    red, ca, cb = m["reduce"], m["a"], m["b"]
+    kd = (red.attr("dims"),) if isinstance(red.attr("dims"), str) else tuple(red.attr("dims"))
+    keep_a = [nm for nm in ca.type.names if nm not in kd]
+    keep_b = [nm for nm in cb.type.names if nm not in kd]
+    out_names = red.type.names
+    riders = [nm for nm in out_names if nm in keep_a and nm in keep_b]
+    mdims = [nm for nm in out_names if nm in keep_a and nm not in riders]
+    ndims = [nm for nm in out_names if nm in keep_b and nm not in riders]
+    if len(riders) > 1:
+        raise Untranslatable("contraction-epilogue: at most one batch (rider) dim on the device")
+    size = {d.name: d for d in red.type.dims}
+    kdim = {nm: ca.type.dim(nm) for nm in kd}
+    # absent groups stand in as unit dims, so the lattice is always (batch, m.., n..)
+    bdim = size[riders[0]] if riders else Dim("_unit_b", 0, 1)
+    if not mdims:
+        size["_unit_m"] = Dim("_unit_m", 0, 1)
+        mdims = ["_unit_m"]
+    if not ndims:
+        size["_unit_n"] = Dim("_unit_n", 0, 1)
+        ndims = ["_unit_n"]
+    if any(kdim[nm].start != 0 for nm in kd):
+        raise Untranslatable("contracted dims must start at 0")
+    return _GemmDims(kd, kdim, riders, bdim, mdims, ndims, size)
+
+
+def _gemm_epilogue(k: Region, m, gd: _GemmDims, y):
+    """(lowered chain, its program over (batch, m, n)) of the epilogue that
+    ends at ``y``; Untranslatable where one program cannot hold it."""
+    red = m["reduce"]
+    if y.type.names and set(y.type.names) != set(red.type.names):
+        raise Untranslatable("the epilogue changes the contraction's lattice")
+    lat = gd.lattice
+    if len(lat) > L.EW_MAX_DIMS:
+        raise Untranslatable(f"an epilogue over {len(lat)} dims (max {L.EW_MAX_DIMS})")
+    scale = 1.0 / math.prod(d.size for d in gd.kdim.values()) if m["f"] == "mean" else None
+    groups = [[0], list(range(1, 1 + len(gd.mdims))), list(range(1 + len(gd.mdims), len(lat)))]
+    try:
+        epi = ewprog.lower(y, lat, {id(p): p for p in k.params}, acc=red, acc_scale=scale)
+        prog = epi.program(_over(y.type.names, y.type.shape, lat),
+                           [_over(op.type.names, op.type.shape, lat) for op in epi.operands])
+        return epi, ewprog.merge_dims(prog, groups)
+    except ewprog.Unlowerable as exc:
+        raise Untranslatable(f"contraction epilogue: {exc}") from None
+
+
 def _chains_as_epilogues(plan, region: Region):
     """``plan`` with each map-chain carve that alone reads one GEMM-shaped
     contraction carve merged into it, as its epilogue (gpt2's gelu(x w + b)
     before the down projection: two launches and a round trip of the wide
     activation less). The partition keeps them apart because the bias
-    broadcast onto the sum counts as a second reader of it."""
+    broadcast onto the sum counts as a second reader of it. A chain that is
+    no epilogue of the contraction (another lattice, or more than one program
+    holds) stays a carve of its own."""
     from .tl.partition import Carve, extract
 
     y = region.body[-1].args[0]
@@ -233,6 +301,10 @@ def _chains_as_epilogues(plan, region: Region):
         kernel, bounds = extract((chain.root,), members)
         m = match_contraction_epilogue(kernel)
         if m is None or m["shape"] != "gemm":
+            continue
+        try:
+            _gemm_epilogue(kernel, m, _gemm_dims(m), kernel.body[-1].args[0])
+        except Untranslatable:
             continue
         group = plan_region(kernel).groups[0]
         merged = Carve(kernel, group, mm.nodes + chain.nodes, chain.root.op, chain.root, bounds, ())
@@ -953,34 +1025,14 @@ class PlanExecutor:
             raise Untranslatable("contraction carve does not match the contraction row")
         if m["shape"] != "gemm":
             return self._reduce(k, m, yroot)
-        red = m["reduce"]
-        kd = (red.attr("dims"),) if isinstance(red.attr("dims"), str) else tuple(red.attr("dims"))
+        gd = _gemm_dims(m)
+        kd, kdim, riders, bdim, mdims, ndims, size = gd.kd, gd.kdim, gd.riders, gd.bdim, gd.mdims, gd.ndims, gd.size
         ca, cb = m["a"], m["b"]
-        keep_a = [nm for nm in ca.type.names if nm not in kd]
-        keep_b = [nm for nm in cb.type.names if nm not in kd]
-        out_names = red.type.names
-        riders = [nm for nm in out_names if nm in keep_a and nm in keep_b]
-        mdims = [nm for nm in out_names if nm in keep_a and nm not in riders]
-        ndims = [nm for nm in out_names if nm in keep_b and nm not in riders]
-        if len(riders) > 1:
-            raise Untranslatable("contraction-epilogue: at most one batch (rider) dim on the device")
-        size = {d.name: d for d in red.type.dims}
-        kdim = {nm: ca.type.dim(nm) for nm in kd}
-        # absent groups stand in as unit dims, so the lattice is always (batch, m.., n..)
-        bdim = size[riders[0]] if riders else Dim("_unit_b", 0, 1)
-        if not mdims:
-            size["_unit_m"] = Dim("_unit_m", 0, 1)
-            mdims = ["_unit_m"]
-        if not ndims:
-            size["_unit_n"] = Dim("_unit_n", 0, 1)
-            ndims = ["_unit_n"]
         B = bdim.size
         M = math.prod(size[nm].size for nm in mdims)
         N = math.prod(size[nm].size for nm in ndims)
         Kx = math.prod(kdim[nm].size for nm in kd)
         KP = -(-Kx // 64) * 64
-        if any(kdim[nm].start != 0 for nm in kd):
-            raise Untranslatable("contracted dims must start at 0")
 
         def pack(core, rows_names, nrows):
             """[B][rows][KP] from the operand chain ``core``."""
@@ -1041,23 +1093,7 @@ class PlanExecutor:
         fuse = rowred is None and self.dtype in ("f32", "bf16")
         pa, pb = pack(ca, mdims, M), pack(cb, ndims, N)
         y = k.body[-1].args[0] if yroot is None else yroot
-        if y.type.names and set(y.type.names) != set(out_names):
-            raise Untranslatable("the epilogue changes the contraction's lattice")
-        lat = (bdim,) + tuple(size[nm] for nm in mdims) + tuple(size[nm] for nm in ndims)
-        if len(lat) > L.EW_MAX_DIMS:
-            raise Untranslatable(f"an epilogue over {len(lat)} dims (max {L.EW_MAX_DIMS})")
-        leaves = {id(p): p for p in k.params}
-        try:
-            epi = ewprog.lower(y, lat, leaves, acc=red, acc_scale=(1.0 / Kx) if m["f"] == "mean" else None)
-        except ewprog.Unlowerable as exc:
-            raise Untranslatable(f"contraction epilogue: {exc}") from None
-        out_st = _over(y.type.names, y.type.shape, lat)
-        prog = epi.program(out_st, [_over(op.type.names, op.type.shape, lat) for op in epi.operands])
-        groups = [[0], list(range(1, 1 + len(mdims))), list(range(1 + len(mdims), len(lat)))]
-        try:
-            prog = ewprog.merge_dims(prog, groups)
-        except ewprog.Unlowerable as exc:
-            raise Untranslatable(f"contraction epilogue: {exc}") from None
+        epi, prog = _gemm_epilogue(k, m, gd, y)
         eslots = tuple(self._index(k, b) for b in epi.bases)
         shape = y.type.shape
         tdt = _TORCH_DT[self.dtype]
