@@ -621,10 +621,18 @@ def contract_views(a: torch.Tensor, a_strides, bt: torch.Tensor, bt_strides, sha
     return out
 
 
+def in_reach(rows: int, k: int, sr: int, sk: int, esize: int) -> bool:
+    """Whether a k slice of ``rows`` x ``k`` elements at these (row, k) strides
+    spans less than the 2 GiB that the contraction kernels' offsets reach
+    (pdh_contract_any and contract_launch refuse it otherwise)."""
+    return (rows + 128) * sr * esize + k * sk * esize < 1 << 31
+
+
 def any_layout(k: int, rows: int, sb: int, sr: int, sk: int) -> bool:
     """Whether :func:`contract_any` reads an operand of ``rows`` rows at these
-    (batch, row, k) element strides: 16-byte chunks along k, or along the rows."""
-    if k % 8 or sb % 8 or min(sb, sr, sk) < 0:
+    (batch, row, k) element strides: 16-byte chunks along k, or along the
+    rows, and a batch entry within the kernels' reach."""
+    if k % 8 or sb % 8 or min(sb, sr, sk) < 0 or not in_reach(rows, k + 64, sr, sk, 2):
         return False
     return (sk == 1 and sr >= k and sr % 8 == 0) or (sr == 1 and sk >= rows and sk % 8 == 0 and rows % 8 == 0)
 

@@ -194,3 +194,55 @@ def test_the_mlp_activation_is_the_up_projections_epilogue(dtype):
     ex = PlanExecutor(plan_model(m.region), m.region, dtype)
     assert [[st.kind for st in n.steps] for n in ex.nested] == [["row-statistics", "contraction-epilogue"]] * 2
     assert all("epilogue=16" in n.steps[1].source for n in ex.nested)
+
+
+@pytest.mark.parametrize("row_major", [False, True])
+def test_an_operand_past_two_gib_is_left_to_the_packing_path(row_major):
+    """any_layout says no exactly where pdh_contract_any refuses the span (its
+    checks come before any launch: nothing runs here)."""
+    from pdum_dsl_amd import _lib as L
+    from pdum_dsl_amd import kernels as K
+
+    def strides(n):  # a weight stored [k][n], or [n][k] with rows padded to 2^20 elements
+        return (0, 1, n) if not row_major else (0, 1 << 20, 1)
+
+    k, lo, hi = 64, 8, 1 << 25
+    while hi - lo > 8:  # the largest n that is read in place
+        mid = (lo + hi) // 16 * 8
+        lo, hi = (mid, hi) if K.any_layout(k, mid, *strides(mid)) else (lo, mid)
+    assert hi == lo + 8 and hi < 10_000_000
+    p = _program(1, 100, hi, False)
+    code = L.lib().pdh_contract_any(4096, 0, 64, 1, 4096, *strides(hi), 1, 100, hi, k, C.byref(p), None, 4096,
+                                    L.PDH_BF16, None, 0, None)
+    assert code == L.PDH_EINVAL and "2 GiB" in L.last_error()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype,N", [("bf16", 10_000_000)])
+def test_the_seat_packs_a_weight_past_two_gib_in_place(dtype, N):
+    """A weight [k][n] whose in-place span is over 2 GiB while its packed rows
+    (k columns each) are under: the packed product."""
+    from pdum_dsl_amd.hip_tile import compile_tile_hip
+    from pdum_dsl_amd.tl import fusion
+    from pdum_dsl_amd.tl.dialect import OPS
+    from pdum_dsl_amd.tl.ir import Builder, Region, tensor_type
+
+    M, Kd = 8, 64
+    bld = Builder(OPS)
+    x, w = bld.param(0, tensor_type(("m", "k"), (M, Kd))), bld.param(1, tensor_type(("k", "n"), (Kd, N)))
+    prod = bld.emit("tl.pointwise", bld.emit("tl.repeat_like", x, w), bld.emit("tl.repeat_like", w, x), f="mul")
+    y = bld.emit("tl.reduce", prod, dims=("k",), f="sum")
+    (grp,) = fusion.plan_region(Region(params=(x, w), body=(bld.emit("core.yield", y),))).groups
+    run = compile_tile_hip(grp.kernel, dtype=dtype)
+    dt = torch.bfloat16
+    g = torch.Generator(device="cuda").manual_seed(1)
+    a = torch.randn(M, Kd, generator=g, device="cuda").to(dt)
+    b = torch.randn(Kd, N, generator=g, device="cuda", dtype=dt)
+    got = run.run_dev([a, b])
+    torch.cuda.synchronize()
+    cols = torch.tensor([0, 1, N // 2 + 1, N - 65, N - 1], device="cuda")
+    ad, bd = a.double().cpu().numpy(), b[:, cols].double().cpu().numpy()
+    want, mag = ad @ bd, np.abs(ad) @ np.abs(bd)
+    # the output's rounding and 64 fp32 products
+    bound = 2.0**-8 * np.abs(want) + 80 * 2.0**-24 * mag
+    assert (np.abs(got[:, cols].double().cpu().numpy() - want) <= bound).all()
