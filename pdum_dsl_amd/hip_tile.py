@@ -753,13 +753,16 @@ def _contraction_runner(region, cb, grid, dtype):
         """Whether the contraction ran on the params where they lie: 16-bit
         through pdh_contract_any, fp32 through pdh_contract_views (its k in
         slices where the output's tiles cannot fill the chip, as the carved-plan
-        executor picks them)."""
+        executor picks them). False where an operand is past the kernels' reach."""
         (sta, stb), shape4 = in_place, (B_, M_, N_, Kdim)
         if dtype != "f32":
             return K.contract_any(a, sta, bt, stb, shape4, prog, ops, out)
         if not split:
             split.append(ewprog.pick_ksplit(prog, B_, M_, N_, KP // 64))
         S, ident, fin = split[0]
+        kc = -(-KP // 64 // S) * 64  # a slice's columns
+        if not (K.in_reach(M_, kc, *sta[1:], 4) and K.in_reach(N_, kc, *stb[1:], 4)):
+            return False
         if S == 1:
             K.contract_views(a, sta, bt, stb, shape4, prog, ops, out)
             return True
