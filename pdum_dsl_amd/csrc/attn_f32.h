@@ -36,8 +36,8 @@ struct AttnF32Args {
 };
 
 // Whether the matrix-core kernels take this geometry: e == od in {64, 128},
-// t and s within 32-bit row arithmetic, and 32 rows of any operand (a staged
-// tile) within the 2 GiB a buffer descriptor's offsets reach.
+// t and s within 32-bit row arithmetic, and the rows of a staged tile (64 at
+// D = 64, 32 at D = 128) within 2 GiB of each other for every operand.
 bool attn_f32_takes(const pdh_attn_geom& g);
 
 // Geometry, mask and scale of `a` (tensor pointers are the caller's to set).

@@ -41,6 +41,11 @@ namespace {
 constexpr float kInf = __builtin_inff();
 constexpr int64_t kMaxRows32 = int64_t{1} << 29;
 
+// The most rows any kernel here stages as one tile, and the row strides (in
+// elements) under which such a tile's byte offsets stay under 2^31.
+constexpr int tile_rows(int64_t D) { return D == 64 ? 64 : 32; }
+constexpr int64_t max_stride(int64_t D) { return (int64_t{1} << 31) / (4 * tile_rows(D)); }
+
 __device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
@@ -65,6 +70,7 @@ struct Tile {
   static constexpr int LD = AL ? 1024 : 256;         // bytes one load instruction of a wave brings
   static constexpr int N = BYTES / LD / W;           // loads per wave
   static_assert(BYTES % (LD * W) == 0, "a tile splits evenly over the waves");
+  static_assert(ROWS <= tile_rows(D), "attn_f32_takes bounds the row strides for this tile");
 
   // rows [row0, row0 + ROWS) of a tensor (rows past `ext` read zeros, or the
   // last row's bytes where rows overlap: callers mask them)
@@ -1070,8 +1076,7 @@ int launch_bwd(AttnF32Args a, int64_t ninst, hipStream_t st) {
 }  // namespace
 
 bool attn_f32_takes(const pdh_attn_geom& g) {
-  const int64_t kMaxStride = int64_t{1} << 24;  // 32 rows of 4-byte elements within 2 GiB
-  auto ok = [&](int64_t st) { return st >= 0 && st < kMaxStride; };
+  auto ok = [&](int64_t st) { return st >= 0 && st < max_stride(g.e); };
   return g.e == g.od && (g.e == 64 || g.e == 128) && g.t <= kMaxRows32 && g.s <= kMaxRows32 && ok(g.q_st) &&
          ok(g.k_st) && ok(g.v_st) && ok(g.o_st) && g.batch * g.heads_q < INT32_MAX / 8;
 }

@@ -39,8 +39,8 @@
 //
 // fp32, the column the reference's f32 Triton runner occupies
 // (conformance/triton_tile.py:662-698): e = od = 64 or 128 run on the fp32
-// matrix cores (attn_f32.hip), e = od = 32 on the row kernel below, any other
-// e, od on the generic kernel (one wave per query row, keys in chunks of 64,
+// matrix cores (attn_f32.hip), e = od = 32 on the row kernel below (and 64
+// where its rows are too far apart for those), any other e, od on the generic kernel (one wave per query row, keys in chunks of 64,
 // one per lane, the same recurrence).
 #include "attn_common.h"
 #include "attn_f32.h"
@@ -698,7 +698,8 @@ __global__ __launch_bounds__(256) void flash_fwd_generic_f32(GenArgs a, int64_t 
   }
 }
 
-// The fp32 kernel for heads of E = OD = 32 features: lane = query
+// The fp32 kernel for heads of E = OD = 32 features (and of 64 where
+// attn_f32_takes refuses the strides): lane = query
 // row, 64 rows per workgroup, so each lane runs its own row's recurrence with
 // no cross-lane reduction, and a key's K and V rows are the same for every
 // lane. The workgroup copies each 64-key chunk of K and V (coalesced rows,
@@ -1060,14 +1061,18 @@ int flash_fwd_impl(const void* q, const void* k, const void* v, void* o, float* 
                G.q_sb, G.q_sh, G.q_st, G.k_sb, G.k_sh, G.k_st, G.v_sb, G.v_sh, G.v_st, G.o_sb, G.o_sh, G.o_st,
                scale, fill, masked, band_lo, band_hi, prune_ok};
     const int64_t nrows = ninst * G.t;
-    if (G.e == G.od && G.e == 32) {  // lanes are rows, K / V rows uniform
+    if (G.e == G.od && (G.e == 32 || G.e == 64)) {  // lanes are rows, K / V rows uniform
       const int64_t nqb = (G.t + 63) / 64;
       PDH_REQUIRE(ninst * nqb <= INT32_MAX && nqb <= INT32_MAX, PDH_EINVAL, "pdh_flash_fwd: too many rows");
       const dim3 grid(static_cast<unsigned>(ninst * nqb));
       static int cus = 0;  // compute units, read once (one device per process)
       if (cus == 0) cus = pdh_device_cus() > 0 ? pdh_device_cus() : 256;
       const bool small = ninst * nqb < cus;  // under one workgroup per compute unit
-      if (small)
+      if (G.e == 64 && small)
+        flash_fwd_rows_f32_lds<64, 64, 8><<<grid, 512, 0, st>>>(ga, static_cast<int>(nqb));
+      else if (G.e == 64)
+        flash_fwd_rows_f32_lds<64, 64, 4><<<grid, 256, 0, st>>>(ga, static_cast<int>(nqb));
+      else if (small)
         flash_fwd_rows_f32_lds<32, 32, 8><<<grid, 512, 0, st>>>(ga, static_cast<int>(nqb));
       else
         flash_fwd_rows_f32_lds<32, 32, 4><<<grid, 256, 0, st>>>(ga, static_cast<int>(nqb));

@@ -130,3 +130,36 @@ def test_strided_and_broadcast_operands():
     for b, hh in ((0, 0), (1, 2)):
         want = cf.attention(*(t[b, hh].double().cpu().numpy() for t in (q, k, v)), scale=0.125)[0]
         np.testing.assert_allclose(r.o[b, hh].double().cpu().numpy(), want, rtol=0, atol=1e-5)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize(
+    "D,stride",
+    [
+        (64, 2**23 - 4),  # the widest rows the matrix-core kernels take: a staged tile spans just under 2 GiB
+        (64, 2**23 - 3),  # the same, rows not 16-byte aligned
+        (64, 2**23),  # past it: the row kernel
+        (128, 2**24 - 4),
+        (128, 2**24),  # past it: the wave-per-row kernel
+    ],
+)
+@pytest.mark.parametrize("H", [2, 40])  # 16-row blocks; 32-row blocks, which stage the longest tiles
+def test_rows_far_apart(D, stride, H):
+    """K rows up to 64 MiB apart (one batch entry of a [rows][batch * heads * D]
+    tensor), NaN between them."""
+    from pdum_dsl_amd import kernels as K
+
+    T, S, Hkv = 224, 67, 2
+    gen = torch.Generator(device="cuda").manual_seed(D + H)
+    q, kc, v = (_tensor(gen, (1, h, n, D), 0) for h, n in ((H, T), (Hkv, S), (Hkv, S)))
+    flat = torch.full(((S - 1) * stride + Hkv * D,), float("nan"), device="cuda")
+    k = flat.as_strided((1, Hkv, S, D), (0, D, stride, 1))
+    k.copy_(kc)
+    got = K.flash_fwd(q, k, v, band=K.Band(None, 0))
+    torch.cuda.synchronize()
+    for hq in (0, H - 1):
+        hk = hq * Hkv // H
+        o, _m, _den, lse = cf.attention(*(t.double().cpu().numpy() for t in (q[0, hq], kc[0, hk], v[0, hk])),
+                                        scale=D**-0.5, band=(None, 0))
+        np.testing.assert_allclose(got.o[0, hq].double().cpu().numpy(), o, rtol=0, atol=1e-5)
+        np.testing.assert_allclose(got.lse[0, hq].double().cpu().numpy(), lse, rtol=0, atol=1e-5)
