@@ -281,9 +281,10 @@ int contract_launch(ContractArgs ca, const pdh_ew_program* epi, const void* cons
   PDH_REQUIRE(ca.rowred < 0 || ca.dtype == PDH_F32, PDH_EUNSUPPORTED, "%s: row partials of fp32 contractions only", fn);
   PDH_REQUIRE(pro == nullptr || (ca.rowred < 0 && (ca.dtype == PDH_F32 || (ca.pro_a && ca.pro_b))), PDH_EUNSUPPORTED,
               "%s: operand prologues: no row partials, and with 16-bit storage both operands computed", fn);
+  const int f32_mode = f32_contract_mode();
   const bool spec = pro != nullptr ? jit_get_pro(*epi, ca.pro_a ? &pro[0].p : nullptr, ca.pro_b ? &pro[1].p : nullptr,
-                                                 fns, lay, ca.dtype)
-                                   : jit_get(JitKind::Contract, *epi, ca.dtype, fns, lay, ca.rowred);
+                                                 fns, lay, ca.dtype, f32_mode)
+                                   : jit_get(JitKind::Contract, *epi, ca.dtype, fns, lay, ca.rowred, f32_mode);
   pdh_ew_program pe = *epi;
   ContractPro pro_a = pro != nullptr ? pro[0] : ContractPro{}, pro_b = pro != nullptr ? pro[1] : ContractPro{};
   void* args3[] = {&ca, &pe, &ops};
@@ -297,7 +298,6 @@ int contract_launch(ContractArgs ca, const pdh_ew_program* epi, const void* cons
     jit_count_launch();
     return PDH_OK;
   };
-  const int f32_mode = f32_contract_mode();
   if (ca.dtype != PDH_F32 && pro != nullptr) {  // 16-bit, computed operands: the one-plane split body
     if (g_cus == 0) g_cus = pdh_device_cus() > 0 ? pdh_device_cus() : 256;
     const bool small = batch * ((m + 127) / 128) * ((n + 127) / 128) < g_cus || m <= 64 || n <= 64 || ca.kp <= 2 * kBK;

@@ -22,6 +22,7 @@
 
 #include "common.h"
 #include "contract_core.h"
+#include "contract_host.h"
 #include "jit.h"
 #include "jit_sources.h"  // generated by the build: the text of dev.h, ew.h, contract_core.h, pdhip.h
 
@@ -67,11 +68,11 @@ void key_program(std::string& k, const pdh_ew_program& p) {
   }
 }
 
-std::string request_key(char what, int dev, int dt, int lay, int red) {
+std::string request_key(char what, int dev, int dt, int lay, int red, int f32_mode) {
   std::string k;
   k.reserve(256);
   k.push_back(what);
-  for (const int v : {dev, dt, lay, red, f32_contract_mode()}) key_add(k, v);
+  for (const int v : {dev, dt, lay, red, f32_mode}) key_add(k, v);
   return k;
 }
 
@@ -197,18 +198,18 @@ std::string gen_eval(const pdh_ew_program& p, int dt, const char* name = "GenEva
   return s;
 }
 
-std::string kernels_src(JitKind kind, int dt, int lay, int red) {
+std::string kernels_src(JitKind kind, int dt, int lay, int red, int f32_mode) {
   const std::string D = dt_name(dt);
   if (kind == JitKind::MapChain)
     return "extern \"C\" __global__ __launch_bounds__(256) void pdh_jit_k0(pdh_ew_program p, pdh::EwOperands ops, "
            "void* out, uint32_t total) { pdh::map_chain_body<" + D + ", 4, pdh::GenEval>(p, ops, out, total); }\n"
            "extern \"C\" __global__ __launch_bounds__(256) void pdh_jit_k1(pdh_ew_program p, pdh::EwOperands ops, "
            "void* out, uint32_t total) { pdh::map_chain_body<" + D + ", 1, pdh::GenEval>(p, ops, out, total); }\n";
-  if (dt == PDH_F32 && f32_contract_mode() == 0)
+  if (dt == PDH_F32 && f32_mode == 0)
     return "extern \"C\" __global__ __launch_bounds__(256) void pdh_jit_k0(pdh::ContractArgs a, pdh_ew_program p, "
            "pdh::EwOperands ops) { pdh::contract_f32_body<pdh::GenEval, " + std::to_string(red) + ">(a, p, ops); }\n";
   if (dt == PDH_F32) {
-    const std::string ns = std::to_string(f32_contract_mode()), nl = ns + ", " + std::to_string(lay);
+    const std::string ns = std::to_string(f32_mode), nl = ns + ", " + std::to_string(lay);
     const std::string rd = ", " + std::to_string(red);
     return "extern \"C\" __global__ __launch_bounds__(256, 2) void pdh_jit_k0(pdh::ContractArgs a, pdh_ew_program p, "
            "pdh::EwOperands ops) { __shared__ __attribute__((aligned(1024))) unsigned char "
@@ -233,8 +234,8 @@ std::string kernels_src(JitKind kind, int dt, int lay, int red) {
 }
 
 // Kernels in a contraction's module.
-int contract_kernels(JitKind kind, int dt) {
-  return kind == JitKind::MapChain ? 2 : (dt != PDH_F32 ? 3 : (f32_contract_mode() != 0 ? 2 : 1));
+int contract_kernels(JitKind kind, int dt, int f32_mode) {
+  return kind == JitKind::MapChain ? 2 : (dt != PDH_F32 ? 3 : (f32_mode != 0 ? 2 : 1));
 }
 
 bool compile_code(const std::string& src, std::vector<char>* code, std::string* err) {
@@ -266,8 +267,8 @@ bool compile_code(const std::string& src, std::vector<char>* code, std::string* 
   return true;
 }
 
-std::string full_source(JitKind kind, const pdh_ew_program& p, int dt, int lay = 0, int red = -1) {
-  return "#include \"contract_core.h\"\n" + gen_eval(p, dt) + kernels_src(kind, dt, lay, red);
+std::string full_source(JitKind kind, const pdh_ew_program& p, int dt, int lay, int red, int f32_mode) {
+  return "#include \"contract_core.h\"\n" + gen_eval(p, dt) + kernels_src(kind, dt, lay, red, f32_mode);
 }
 
 std::string reduce_source(const pdh_ew_program& ps, const pdh_ew_program& pe, int dt) {
@@ -284,8 +285,9 @@ std::string reduce_source(const pdh_ew_program& ps, const pdh_ew_program& pe, in
 
 // The fp32 contraction with operand prologues: the epilogue's evaluator, one
 // per computed operand (GenProA, GenProB; an absent one is a stub the kernel
-// never calls) and the prologue kernels of the current fp32 mode.
-std::string pro_source(const pdh_ew_program& pe, const pdh_ew_program* pa, const pdh_ew_program* pb, int lay, int dt) {
+// never calls) and the prologue kernels of the fp32 mode.
+std::string pro_source(const pdh_ew_program& pe, const pdh_ew_program* pa, const pdh_ew_program* pb, int lay, int dt,
+                       int f32_mode) {
   const char* stub = "namespace pdh {\nstruct %s {\n  static constexpr bool kVec = false;\n  static constexpr int "
                      "kStoreRun = 16;\n  template <int EPT>\n  static __device__ __forceinline__ void run(const "
                      "pdh_ew_program&, const EwOperands&, int, const int (&)[PDH_EW_MAX_DIMS], const float (&)[EPT], "
@@ -301,11 +303,11 @@ std::string pro_source(const pdh_ew_program& pe, const pdh_ew_program* pa, const
                   (pb ? gen_eval(*pb, dt, "GenProB") : stub_of("GenProB"));
   const std::string args = "(pdh::ContractArgs a, pdh_ew_program p, pdh::EwOperands ops, pdh::ContractPro pa, "
                            "pdh::ContractPro pb)";
-  if (dt == PDH_F32 && f32_contract_mode() == 0)
+  if (dt == PDH_F32 && f32_mode == 0)
     return s + "extern \"C\" __global__ __launch_bounds__(256) void pdh_jit_k0" + args +
            " { pdh::contract_f32_body<pdh::GenEval, -1, pdh::GenProA, pdh::GenProB, true>(a, p, ops, &pa, &pb); }\n";
   // 16-bit storage: one bf16 plane (the operands' values rounded to bf16)
-  const int ns = dt == PDH_F32 ? f32_contract_mode() : 1;
+  const int ns = dt == PDH_F32 ? f32_mode : 1;
   const std::string nl = std::to_string(ns) + ", " + std::to_string(lay);
   std::string k;
   for (int small = 0; small < 2; ++small) {
@@ -377,17 +379,18 @@ bool get(const std::string& key, int dev, const std::string& src, int count, hip
 
 // The specialized kernels for program p (jit.h), or false when the
 // interpreter must run it.
-bool jit_get(JitKind kind, const pdh_ew_program& p, int dt, hipFunction_t fns[kJitFns], int lay, int red) {
+bool jit_get(JitKind kind, const pdh_ew_program& p, int dt, hipFunction_t fns[kJitFns], int lay, int red,
+             int f32_mode) {
   if (!jit_enabled()) return false;
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess) return false;
-  std::string key = request_key(kind == JitKind::MapChain ? 'm' : 'c', dev, dt, lay, red);
+  std::string key = request_key(kind == JitKind::MapChain ? 'm' : 'c', dev, dt, lay, red, f32_mode);
   key_program(key, p);
   bool known;
   const bool found = find_request(key, fns, &known);
   return known ? found
-               : get(key, dev, full_source(kind, p, dt, lay, red),
-                     contract_kernels(kind, dt), fns);
+               : get(key, dev, full_source(kind, p, dt, lay, red, f32_mode), contract_kernels(kind, dt, f32_mode),
+                     fns);
 }
 
 // The specialized row-reduce kernels for (summand, epilogue): fns[0] one
@@ -396,7 +399,7 @@ bool jit_get_reduce(const pdh_ew_program& ps, const pdh_ew_program& pe, int dt, 
   if (!jit_enabled()) return false;
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess) return false;
-  std::string key = request_key('r', dev, dt, 0, 0);
+  std::string key = request_key('r', dev, dt, 0, 0, 0);
   key_program(key, ps);
   key_program(key, pe);
   bool known;
@@ -408,18 +411,18 @@ bool jit_get_reduce(const pdh_ew_program& ps, const pdh_ew_program& pe, int dt, 
 // 128 x 128-tile kernel (or the VALU one in fp32 mode 0), fns[1] the
 // 64 x 64-tile one; or false.
 bool jit_get_pro(const pdh_ew_program& pe, const pdh_ew_program* pa, const pdh_ew_program* pb, hipFunction_t fns[kJitFns],
-                 int lay, int dt) {
+                 int lay, int dt, int f32_mode) {
   if (!jit_enabled()) return false;
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess) return false;
-  std::string key = request_key('p', dev, dt, lay, (pa != nullptr ? 1 : 0) | (pb != nullptr ? 2 : 0));
+  std::string key = request_key('p', dev, dt, lay, (pa != nullptr ? 1 : 0) | (pb != nullptr ? 2 : 0), f32_mode);
   key_program(key, pe);
   if (pa != nullptr) key_program(key, *pa);
   if (pb != nullptr) key_program(key, *pb);
   bool known;
   const bool found = find_request(key, fns, &known);
-  return known ? found : get(key, dev, pro_source(pe, pa, pb, lay, dt),
-                           dt != PDH_F32 || f32_contract_mode() != 0 ? 2 : 1, fns);
+  return known ? found : get(key, dev, pro_source(pe, pa, pb, lay, dt, f32_mode),
+                           dt != PDH_F32 || f32_mode != 0 ? 2 : 1, fns);
 }
 
 void jit_count_launch() { ++g_launched; }
@@ -446,7 +449,8 @@ extern "C" size_t pdh_ew_jit_source(const pdh_ew_program* prog, int kind, int dt
       kind < 0 || kind > 7)
     return 0;
   const std::string src = full_source(kind == 0 ? JitKind::MapChain : JitKind::Contract, *prog, dtype,
-                                      kind > 1 && kind < 5 ? kind - 1 : 0, kind >= 5 ? kind - 5 : -1);
+                                      kind > 1 && kind < 5 ? kind - 1 : 0, kind >= 5 ? kind - 5 : -1,
+                                      f32_contract_mode());
   if (buf && n) {
     const size_t k = src.size() < n - 1 ? src.size() : n - 1;
     std::memcpy(buf, src.data(), k);
@@ -462,7 +466,8 @@ extern "C" int pdh_ew_jit_compile(const pdh_ew_program* prog, int kind, int dtyp
   std::vector<char> code;
   std::string err;
   PDH_REQUIRE(compile_code(full_source(kind == 0 ? JitKind::MapChain : JitKind::Contract, *prog, dtype,
-                                       kind > 1 && kind < 5 ? kind - 1 : 0, kind >= 5 ? kind - 5 : -1),
+                                       kind > 1 && kind < 5 ? kind - 1 : 0, kind >= 5 ? kind - 5 : -1,
+                                      f32_contract_mode()),
                            &code, &err),
               PDH_ELAUNCH, "%s", err.c_str());
   return PDH_OK;
