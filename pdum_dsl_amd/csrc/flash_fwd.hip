@@ -668,8 +668,9 @@ __global__ __launch_bounds__(256) void flash_fwd_generic_f32(GenArgs a, int64_t 
       }
     }
     const float mnew = fmaxf(m, wave_max(sc));
-    const float alpha = __expf(m - mnew);
-    const float p = key < a.s ? __expf(sc - mnew) : 0.f;
+    const float ref = mnew == -kInf ? 0.f : mnew;  // only scores of -inf so far: they weigh 0, not NaN
+    const float alpha = __expf(m - ref);
+    const float p = key < a.s ? __expf(sc - ref) : 0.f;
     l = l * alpha + wave_sum(p);
     m = mnew;
 #pragma unroll

@@ -115,6 +115,31 @@ def test_a_pruned_window_is_bit_equal_to_the_full_sweep(B, H, T, S, D):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("fill", [float("-inf"), torch.finfo(torch.float32).min], ids=["-inf", "lowest"])
+@pytest.mark.parametrize("H,T,S,D", [(2, 130, 321, 64), (40, 224, 300, 64), (2, 130, 321, 128), (3, 70, 200, 32), (2, 70, 200, 40)])
+def test_the_lowest_fills_leave_live_rows_finite(H, T, S, D, fill):
+    """Whole tiles a row sees only as masked, with fills whose score is -inf or
+    the lowest value, on the matrix-core, row and generic kernels: they add
+    nothing, pruned or not."""
+    from pdum_dsl_amd import kernels as K
+
+    gen = torch.Generator(device="cuda").manual_seed(D + T)
+    q = _tensor(gen, (1, H, T, D), 0)
+    k, v = (_tensor(gen, (1, H, S, D), 0) for _ in range(2))
+    band = (65, 120)  # the last rows' first live key is past three 64-key chunks
+    if T + band[0] > S:
+        band = (65 - T, 10)
+    outs = [K.flash_fwd(q, k, v, band=K.Band(*band), fill=fill, prune=p) for p in (True, False)]
+    torch.cuda.synchronize()
+    for out in outs:
+        for h in (0, H - 1):
+            x = [t[0, h].double().cpu().numpy() for t in (q, k, v)]
+            o, _m, _den, lse = cf.attention(*x, scale=D**-0.5, band=band)
+            np.testing.assert_allclose(out.o[0, h].double().cpu().numpy(), o, rtol=0, atol=1e-5)
+            np.testing.assert_allclose(out.lse[0, h].double().cpu().numpy(), lse, rtol=0, atol=1e-5)
+
+
+@pytest.mark.gpu
 def test_strided_and_broadcast_operands():
     """Rows of a wider tensor (a stride that is no multiple of four), heads
     behind rows, and K / V rows repeated by a zero stride."""
