@@ -36,28 +36,50 @@ def _tensor(gen, shape, offset):
     return flat[offset:].view(shape)
 
 
+# (B, Hq, Hkv, T, S, D, band): (rows of a forward block, rows of a backward block) the launcher picks
+CASES = {
+    # the smallest, one short tile each
+    (1, 1, 1, 1, 1, 64, None): (16, 16),
+    (1, 1, 1, 15, 17, 128, (None, 2)): (16, 16),
+    # 16-row blocks, keys over the waves (forward) and rings (backward)
+    (1, 2, 1, 100, 333, 64, (-70, 240)): (16, 16),
+    (1, 3, 3, 65, 64, 128, (None, -1)): (16, 16),  # a fully masked row: no prune
+    (2, 4, 1, 130, 130, 128, (None, 0)): (16, 16),  # a group's key blocks sweep four heads
+    (2, 40, 40, 95, 95, 128, None): (16, 64),
+    # 32-row blocks, two waves on the keys
+    (2, 32, 8, 150, 270, 64, (None, 120)): (32, 16),
+    (2, 40, 40, 128, 95, 128, None): (32, 64),
+    (1, 40, 20, 201, 310, 128, (-30, 140)): (32, 16),
+    # 64-row blocks
+    (4, 64, 32, 100, 65, 64, (-20, None)): (64, 64),
+    (4, 64, 32, 100, 65, 128, (None, 9)): (64, 64),
+    # 128-row blocks of eight waves
+    (4, 64, 32, 129, 65, 64, (-20, 3)): (128, 64),
+    (8, 64, 64, 129, 65, 64, (None, 0)): (128, 64),
+    (8, 64, 16, 70, 97, 128, (-60, None)): (128, 64),
+}
+
+
+def _block_rows(B, Hq, Hkv, T, S, D, cus=256):
+    """launch_fwd's and launch_bwd's choice (attn_f32.hip)."""
+    q = lambda rows: B * Hq * -(-T // rows)  # noqa: E731
+    fwd = 128 if q(128) >= 2 * cus else 64 if q(64) >= 2 * cus else 32 if q(32) >= cus else 16
+    limit = 2 * cus if D == 64 or Hq > Hkv else 3 * cus // 4
+    return fwd, 16 if q(64) + B * Hkv * -(-S // 64) < limit else 64
+
+
+def test_the_cases_reach_every_block_shape():
+    reached = set()
+    for (*shape, _band), want in CASES.items():
+        assert _block_rows(*shape) == want, shape
+        reached |= {(shape[-1], "forward", want[0]), (shape[-1], "backward", want[1])}
+    assert reached == {(D, *x) for D in (64, 128) for x in (("forward", 16), ("forward", 32), ("forward", 64),
+                                                            ("forward", 128), ("backward", 16), ("backward", 64))}
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("offset", [0, 1])
-@pytest.mark.parametrize(
-    "B,Hq,Hkv,T,S,D,band",
-    [
-        # the smallest, one short tile each
-        (1, 1, 1, 1, 1, 64, None),
-        (1, 1, 1, 15, 17, 128, (None, 2)),
-        # 16-row blocks, keys over the waves (forward) and rings (backward)
-        (1, 2, 1, 100, 333, 64, (-70, 240)),
-        (1, 3, 3, 65, 64, 128, (None, -1)),  # a fully masked row: no prune
-        (2, 4, 1, 130, 130, 128, (None, 0)),  # a group's key blocks sweep four heads
-        # 32-row blocks, two waves on the keys; 64-row backward blocks
-        (2, 32, 8, 150, 270, 64, (None, 120)),
-        (2, 40, 40, 95, 95, 128, None),
-        # 64-row blocks
-        (4, 64, 32, 129, 65, 64, (-20, 3)),
-        # 128-row blocks of eight waves
-        (8, 64, 64, 129, 65, 64, (None, 0)),
-        (8, 64, 16, 70, 97, 128, (-60, None)),
-    ],
-)
+@pytest.mark.parametrize("B,Hq,Hkv,T,S,D,band", CASES)
 def test_forward_and_backward_match_the_closed_forms(B, Hq, Hkv, T, S, D, band, offset):
     """Sampled (batch, K / V head) groups, every query head of each: 1e-5 of
     scale, the fp32 bound of the other attention tests (sums of at most a few
@@ -97,7 +119,8 @@ def test_forward_and_backward_match_the_closed_forms(B, Hq, Hkv, T, S, D, band, 
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("B,H,T,S,D", [(1, 2, 70, 400, 64), (2, 32, 100, 300, 128), (8, 64, 129, 200, 64)])
+@pytest.mark.parametrize("B,H,T,S,D", [(1, 2, 70, 400, 64), (2, 32, 100, 300, 128), (4, 64, 100, 190, 64),
+                                       (4, 64, 100, 190, 128), (8, 64, 129, 200, 64)])
 def test_a_pruned_window_is_bit_equal_to_the_full_sweep(B, H, T, S, D):
     """A window leaves dead keys on both sides of a block's range; in the full
     sweep their fill scores must vanish from every state."""
