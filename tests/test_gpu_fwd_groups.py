@@ -43,30 +43,53 @@ def _exact(q, k, v, band, fill, scale):
     return torch.matmul(p, v), torch.matmul(p, v.abs()), size, torch.logsumexp(s, -1)
 
 
+# (B, H, Hkv, T, S, D, band): the (row, key) wave groups of the workgroup the launcher picks
+CASES = {
+    (1, 1, 1, 1, 1024, 64, None): (2, 4),
+    (1, 2, 1, 65, 1055, 64, (None, 990)): (2, 4),
+    (1, 3, 3, 1030, 1024, 64, (None, 0)): (2, 4),
+    (1, 2, 2, 63, 256, 64, None): (2, 2),
+    (1, 4, 1, 130, 321, 64, (None, 2)): (2, 2),
+    (2, 2, 1, 200, 1500, 64, (-300, 5)): (2, 2),  # a window: fewer live keys than stored
+    (1, 1, 1, 33, 257, 128, (None, -1)): (2, 2),  # a fully masked row: no prune
+    (1, 8, 2, 300, 417, 128, (None, 0)): (2, 2),
+    (1, 6, 6, 129, 300, 128, (120, None)): (2, 2),
+    (3, 24, 12, 190, 287, 128, None): (4, 2),
+    # uneven sweeps over more blocks than compute units: up to 1.5 a unit at 512 keys ...
+    (1, 100, 100, 257, 515, 64, (None, 100)): (2, 2),
+    (1, 100, 50, 257, 515, 128, (None, 100)): (2, 2),
+    # ... and up to 4 (D = 64) or 2 (128) at 2048 keys
+    (1, 36, 36, 2048, 2048, 64, (None, 0)): (2, 2),
+    (1, 200, 100, 129, 2050, 128, (None, 1900)): (2, 2),
+    # past those lines: one key group
+    (2, 70, 70, 257, 515, 64, (None, 100)): (4, 1),
+    (1, 100, 50, 400, 513, 128, (None, 0)): (4, 1),
+}
+
+
+def _workgroup(B, H, Hkv, T, S, D, band, cus=256):
+    """launch_mfma's choice (flash_fwd.hip)."""
+    blocks, (lo, hi) = B * H * -(-T // 128), band or (None, None)
+    keys = S if lo is None or hi is None else min(S, hi - lo + 128)
+    uneven = (lo is None) != (hi is None)
+    if blocks <= cus and keys >= 256:
+        if D == 64 and 2 * blocks <= cus and keys >= 1024:
+            return 2, 4
+        return (4, 2) if D == 128 and 2 * blocks > cus and not uneven else (2, 2)
+    wide = (2 * blocks <= 3 * cus and keys >= 512) or (blocks <= (4 if D == 64 else 2) * cus and keys >= 2048)
+    return (2, 2) if uneven and wide else (4, 1)
+
+
+def test_the_cases_reach_every_workgroup_shape():
+    for case, want in CASES.items():
+        assert _workgroup(*case) == want, case
+    assert {(c[5], w) for c, w in CASES.items()} == {(64, (2, 4)), (64, (2, 2)), (64, (4, 1)), (128, (2, 2)), (128, (4, 2)),
+                                                     (128, (4, 1))}
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("dt", ["bfloat16", "float16"])
-@pytest.mark.parametrize(
-    "B,H,Hkv,T,S,D,band",
-    [
-        # four key groups, 64-row blocks
-        (1, 1, 1, 1, 1024, 64, None),
-        (1, 2, 1, 65, 1055, 64, (None, 990)),
-        (1, 3, 3, 1030, 1024, 64, (None, 0)),
-        # two key groups, 64-row blocks
-        (1, 2, 2, 63, 256, 64, None),
-        (1, 4, 1, 130, 321, 64, (None, 2)),
-        (2, 2, 1, 200, 1500, 64, (-300, 5)),  # a window: fewer live keys than stored
-        (1, 1, 1, 33, 257, 128, (None, -1)),  # a fully masked row: no prune
-        (1, 8, 2, 300, 417, 128, (None, 0)),
-        (1, 6, 6, 129, 300, 128, (120, None)),
-        # two key groups, 128-row blocks
-        (3, 24, 12, 190, 287, 128, None),
-        # uneven sweeps over more blocks than compute units
-        (2, 70, 70, 257, 515, 64, (None, 100)),
-        (1, 36, 36, 2048, 2048, 64, (None, 0)),
-        (1, 100, 50, 400, 513, 128, (None, 0)),
-    ],
-)
+@pytest.mark.parametrize("B,H,Hkv,T,S,D,band", CASES)
 def test_grouped_keys_match_float64(B, H, Hkv, T, S, D, band, dt):
     from pdum_dsl_amd import kernels as K
 
