@@ -213,10 +213,10 @@ def test_flash_fwd_fp32_generic_matches_oracle(K, T, S, E, OD, causal):
      (4, 16, 8, 1024, 1024, 64, (None, 0)), (2, 32, 32, 500, 700, 32, None)],
 )
 def test_flash_fwd_fp32_row_kernel_matches_oracle(K, B, Hq, Hkv, T, S, D, band):
-    """e = od = 32 or 64 at fp32 take the row kernel (lane = query row, K / V
-    chunks staged through LDS, the key range split over eight waves on grids
-    under one workgroup per CU, four on the last two cases' larger grids):
-    causal, windowed, half-open and fully-masked-row bands (the last disables
+    """e = od = 32 at fp32 takes the row kernel (lane = query row, K / V chunks
+    staged through LDS, the key range split over eight waves on grids under
+    one workgroup per CU, four on the last case's larger grid), 64 the
+    matrix-core ones: causal, windowed, half-open and fully-masked-row bands (the last disables
     the prune), grouped heads, row and key tails, the artifacts."""
     rng = np.random.default_rng(T * 7 + S + D)
     q, k, v = _qkv(rng, B, Hq, Hkv, T, S, D, D, torch.float32)
@@ -237,12 +237,14 @@ def test_pruned_sweep_is_bit_equal_to_the_full_sweep(K, dtype):
     assert torch.equal(full.m, pruned.m) and torch.equal(full.den, pruned.den)
 
 
+@pytest.mark.parametrize("D", [32, 64])
 @pytest.mark.parametrize("B,H,T", [(1, 2, 320), (8, 32, 256)])
-def test_the_row_kernel_prunes_bit_exactly(K, B, H, T):
-    """The fp32 row kernel at both wave counts (a grid under one workgroup
-    per CU, and one over): a causal prune leaves every bit as the full sweep."""
+def test_the_row_kernel_prunes_bit_exactly(K, B, H, T, D):
+    """The fp32 row kernel (D = 32) at both wave counts (a grid under one
+    workgroup per CU, and one over), and the matrix-core kernels (64): a causal
+    prune leaves every bit as the full sweep."""
     rng = np.random.default_rng(12)
-    q, k, v = _qkv(rng, B, H, H, T, T, 64, 64, torch.float32)
+    q, k, v = _qkv(rng, B, H, H, T, T, D, D, torch.float32)
     full = K.flash_fwd(q, k, v, band=K.CAUSAL, prune=False, want_artifacts=True)
     pruned = K.flash_fwd(q, k, v, band=K.CAUSAL, prune=True, want_artifacts=True)
     torch.cuda.synchronize()
