@@ -27,8 +27,8 @@
 // -> 163 us and forward 182 -> 58 us; 32 heads x 2048, D = 64, all keys live:
 // forward 119 TFLOP/s, backward 109 (seven products, the dQ role recomputes
 // two) of the 157 the fp32 matrix cores peak at; one head x 256: 29 -> 7.3 us.
-// The distance to 64 bits is the VALU kernels' or smaller (o 1.8e-7, dK 8e-7 of
-// the norm at 24 x 1000).
+// The distance to 64 bits is smaller than the VALU kernels' (o 1.8e-7, dK 3.9e-7 of
+// the norm at 24 x 1000, against 2.6e-7 and 8.1e-7).
 #include "attn_f32.h"
 
 #include "attn_common.h"
@@ -538,9 +538,17 @@ __device__ __forceinline__ void sweep_range(const AttnF32Args& a, int o0, int ex
 // sweeps query tiles (Q, dO and their statistics in LDS):
 //   S = Q K^T, dP = dO V^T - delta, P = exp2(S scale log2(e) - lse2), dS = P dP
 //   dV^T += dO^T P, dK^T += Q^T dS
+// Short chains of sums, as in the forward: the even and the odd chunks of D
+// apart, and each tile's products added to the gradient as a whole. With one
+// chain over D and one over the swept rows the gradients were 1-6% further from
+// 64 bits than the VALU kernels' (24 causal heads x 1000, D = 64: dQ 5.1e-7, dK
+// 8.2e-7, dV 8.1e-7 of the norm; the VALU's 5.0, 8.1, 8.0; so 3.7, 3.9, 3.4) and
+// the kernel 0-5% faster at D = 64 (that shape 154 us both ways, 24 heads x 2000,
+// all keys live, 757 -> 791), 2% faster to 25% slower at D = 128 (64 heads x 700
+// in a window 185 -> 189; 32 heads over 8 x 1024 causal 960 -> 740).
 template <int D, bool AL>
 __device__ __forceinline__ void bwd_dkdv(const AttnF32Args& a, int inst_kv, int kb, unsigned char* smem) {
-  constexpr int NS = D / 16;
+  constexpr int NS = D / 16, FG = D == 64 ? 4 : 2;  // FG: feature blocks whose tile sums are in flight
   using T = Tile<D, 32, kBW, AL>;
   using L = BwdLds<D>;
   const int lane = threadIdx.x & 63, w = wave_id(), c = lane & 15, G = lane >> 4;
@@ -581,10 +589,10 @@ __device__ __forceinline__ void bwd_dkdv(const AttnF32Args& a, int inst_kv, int 
     const unsigned char* qt_ = smem + buf * 2 * L::TB;
     const unsigned char* ot_ = qt_ + L::TB;
     const float* stat = reinterpret_cast<const float*>(smem + L::STAT + buf * 3 * 256);
-    f32x4 s[2], p[2];
+    f32x4 s[2], p[2], s1[2], p1[2];  // even and odd chunks of D apart, as in the forward
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      s[h] = f32x4{0.f, 0.f, 0.f, 0.f};
+      s[h] = s1[h] = p1[h] = f32x4{0.f, 0.f, 0.f, 0.f};
       p[h] = *reinterpret_cast<const f32x4*>(stat + 16 * h + 4 * G);  // -delta
     }
 #pragma unroll
@@ -599,9 +607,15 @@ __device__ __forceinline__ void bwd_dkdv(const AttnF32Args& a, int inst_kv, int 
       for (int j = 0; j < 4; ++j)
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
-          s[h] = mfma4(qf[h][j], kf[x][j], s[h]);
-          p[h] = mfma4(of[h][j], vf[x][j], p[h]);
+          f32x4 &t = x & 1 ? s1[h] : s[h], &u = x & 1 ? p1[h] : p[h];
+          t = mfma4(qf[h][j], kf[x][j], t);
+          u = mfma4(of[h][j], vf[x][j], u);
         }
+    }
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      s[h] += s1[h];
+      p[h] += p1[h];
     }
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
@@ -625,14 +639,26 @@ __device__ __forceinline__ void bwd_dkdv(const AttnF32Args& a, int inst_kv, int 
       }
     }
 #pragma unroll
-    for (int h = 0; h < 2; ++h)
+    for (int f0 = 0; f0 < NS; f0 += FG) {
+      f32x4 tv[FG], tk[FG];
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
+      for (int f = 0; f < FG; ++f) tv[f] = tk[f] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int f = 0; f < NS; ++f) {
-          dv[f] = mfma4(off.feature(ot_, h, f, j), s[h][j], dv[f]);
-          dk[f] = mfma4(off.feature(qt_, h, f, j), p[h][j], dk[f]);
-        }
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+          for (int f = 0; f < FG; ++f) {
+            tv[f] = mfma4(off.feature(ot_, h, f0 + f, j), s[h][j], tv[f]);
+            tk[f] = mfma4(off.feature(qt_, h, f0 + f, j), p[h][j], tk[f]);
+          }
+#pragma unroll
+      for (int f = 0; f < FG; ++f) {
+        dv[f0 + f] += tv[f];
+        dk[f0 + f] += tk[f];
+      }
+      if constexpr (D == 128) __builtin_amdgcn_sched_barrier(0);  // keeps the next group's reads out: else 73 spills
+    }
   };
 
   // items (query head of the group, tile), head-major; the staging cursor runs one item ahead
@@ -714,10 +740,10 @@ __device__ __forceinline__ void bwd_dq(const AttnF32Args& a, int inst, int qb, u
     }
     const unsigned char* kt_ = smem + buf * 2 * L::TB;
     const unsigned char* vt_ = kt_ + L::TB;
-    f32x4 s[2], p[2];
+    f32x4 s[2], p[2], s1[2], p1[2];
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      s[h] = f32x4{0.f, 0.f, 0.f, 0.f};
+      s[h] = s1[h] = p1[h] = f32x4{0.f, 0.f, 0.f, 0.f};
       p[h] = f32x4{ndelta, ndelta, ndelta, ndelta};
     }
 #pragma unroll
@@ -732,9 +758,15 @@ __device__ __forceinline__ void bwd_dq(const AttnF32Args& a, int inst, int qb, u
       for (int j = 0; j < 4; ++j)
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
-          s[h] = mfma4(kf[h][j], qf[x][j], s[h]);
-          p[h] = mfma4(vf[h][j], of[x][j], p[h]);
+          f32x4 &t = x & 1 ? s1[h] : s[h], &u = x & 1 ? p1[h] : p[h];
+          t = mfma4(kf[h][j], qf[x][j], t);
+          u = mfma4(vf[h][j], of[x][j], u);
         }
+    }
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      s[h] += s1[h];
+      p[h] += p1[h];
     }
 #pragma unroll
     for (int h = 0; h < 2; ++h)
@@ -750,11 +782,19 @@ __device__ __forceinline__ void bwd_dq(const AttnF32Args& a, int inst, int qb, u
         }
     }
 #pragma unroll
-    for (int h = 0; h < 2; ++h)
+    for (int f0 = 0; f0 < NS; f0 += 4) {
+      f32x4 tq[4];
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
+      for (int f = 0; f < 4; ++f) tq[f] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int f = 0; f < NS; ++f) dq[f] = mfma4(off.feature(kt_, h, f, j), p[h][j], dq[f]);
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+          for (int f = 0; f < 4; ++f) tq[f] = mfma4(off.feature(kt_, h, f0 + f, j), p[h][j], tq[f]);
+#pragma unroll
+      for (int f = 0; f < 4; ++f) dq[f0 + f] += tq[f];
+    }
   };
   auto step = [&](int kt, auto bufc) __attribute__((always_inline)) {
     wait_vmcnt0();
@@ -1054,11 +1094,14 @@ int launch_bwd(AttnF32Args a, int64_t ninst, hipStream_t st) {
   };
   // Under two 64-row blocks per compute unit the longest block sets the time:
   // 16-row blocks are four times as many and a quarter as long (forward +
-  // backward, D = 64: 4 heads x 1024 rows, 128 blocks, 101 -> 70 us; 12 x 512,
-  // 192 blocks, 65 -> 60; 12 x 1024, 384 blocks, 159 -> 154; but 24 x 1000, 768
-  // blocks, 206 -> 213). At D = 128 their rings leave one wave per SIMD, so the
-  // line is lower (16 heads x 512, 256 blocks, 113 -> 123 us) unless a group's
-  // heads make the key blocks long (16 heads over 4, 738 rows, 494 -> 324).
+  // backward, causal, D = 64: 4 heads x 1024 rows, 128 blocks, 102 -> 67 us; 12 x
+  // 512, 192 blocks, 64 -> 56; 12 x 1024, 384 blocks, 163 -> 154; but 16 x 1024, 512
+  // blocks, 165 -> 176 and 24 x 1000, 768 blocks, 206 -> 212). At D = 128 their
+  // rings leave one wave per SIMD, so the line is lower (8 heads x 512, 128 blocks,
+  // 98 -> 74; 12 x 512, 192 blocks, 110 -> 106; 16 x 512, 256 blocks, 114 -> 125)
+  // unless a group's heads make the key blocks long (heads over 4: 16 x 738, 240
+  // blocks, 495 -> 327; 32 over 8 x 738, 480 blocks, 546 -> 461; x 1024, 640 blocks,
+  // 853 -> 866).
   int64_t nblk = blocks(kBO);
   const bool small = nblk < (D == 64 || a.group > 1 ? 2 * cus : 3 * cus / 4);
   if (small) nblk = blocks(16);

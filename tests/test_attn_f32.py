@@ -119,6 +119,35 @@ def test_forward_and_backward_match_the_closed_forms(B, Hq, Hkv, T, S, D, band, 
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize(
+    "B,H,T,D,band,bound",
+    [
+        (2, 12, 1000, 64, (None, 0), (4.97e-7, 8.13e-7, 8.04e-7)),
+        (2, 32, 700, 128, (-200, 0), (5.38e-7, 5.77e-7, 5.20e-7)),
+    ],
+)
+def test_gradients_stay_as_close_to_64_bits_as_fp32_sums_in_order(B, H, T, D, band, bound):
+    """The 64-row backward's relative errors (2-norm) of dQ, dK, dV against
+    float64: no larger than those of the fp32 VALU kernels (bwd_rows_f32), one
+    running sum per element, measured on inputs of this distribution."""
+    from pdum_dsl_amd import kernels as K
+
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    q, k, v, do = (_tensor(gen, (B, H, T, D), 0) for _ in range(4))
+    fw = K.flash_fwd(q, k, v, band=K.Band(*band))
+    got = K.flash_bwd(q, k, v, fw.o, do, fw.lse, band=K.Band(*band))
+    torch.cuda.synchronize()
+    err, size = np.zeros(3), np.zeros(3)
+    for b in range(B):
+        for h in range(0, H, 5):
+            x = [t[b, h].double().cpu().numpy() for t in (q, k, v, do)]
+            for i, want in enumerate(cf.attention_bwd(*x, scale=D**-0.5, band=band)):
+                err[i] += ((got[i][b, h].double().cpu().numpy() - want) ** 2).sum()
+                size[i] += (want**2).sum()
+    assert (np.sqrt(err / size) <= bound).all(), np.sqrt(err / size)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("B,H,T,S,D", [(1, 2, 70, 400, 64), (2, 32, 100, 300, 128), (4, 64, 100, 190, 64),
                                        (4, 64, 100, 190, 128), (8, 64, 129, 200, 64)])
 def test_a_pruned_window_is_bit_equal_to_the_full_sweep(B, H, T, S, D):
