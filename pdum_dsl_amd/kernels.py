@@ -353,24 +353,43 @@ def pick_fwd_splits(ninst: int, t: int, s: int, cus: int | None = None) -> int:
     return int(max(1, min(ntiles // 8, (3 * cus) // blocks, 64)))
 
 
+def _one_launch_keys(blocks: float, d: int) -> float:
+    """Live keys a row under which one launch whose waves share the keys inside
+    a workgroup (launch_mfma in flash_fwd.hip) is the faster forward of
+    ``blocks`` 128-row blocks on 256 compute units; above, ``pick_fwd_splits``'
+    workgroups and their combine are. One launch's time grows with the keys
+    alone until two of its workgroups share a unit, a split's with blocks x
+    keys. Measured (bf16, heads x t x keys, us, one launch / split): d = 64,
+    1 x 1024 x 1024 11.6 / 16.4, x 3000 23.2 / 17.3, x 6000 39 / 26; 4 x 1024 x
+    3000 23.1 / 22.5, x 6000 39 / 34; 12 x 1024 x 4096 28 / 31, x 6000 39 / 37;
+    4 x 4177 causal 40 / 35; 6 x 3000 x 3000 35 / 31; 24 x 1024 x 3000 35 / 35,
+    x 6000 63 / 54; 16 x 2048 x 6000 65 / 66. d = 128, 1 x 1024 x 1024 17.8 /
+    16.6, x 3000 42 / 22; 8 x 1024 x 3000 42 / 39; 24 x 1024 x 3000 52 / 57, x
+    6000 94 / 87; 16 x 2048 x 6000 98 / 108."""
+    if d == 64:  # to 128 blocks eight waves on 64 rows, four key groups; past them two
+        return 2000 if blocks <= 24 else (3400 + 22 * blocks if blocks <= 128 else 30 * blocks - 2000)
+    return max(900, 30 * blocks) if blocks <= 128 else 30 * blocks - 1300
+
+
 def _fwd_splits(ninst: int, t: int, s: int, d: int, band: Band | None, cus: int | None = None) -> int:
-    """Key splits of a forward that names none: 1 where one launch whose waves
-    share the keys inside a workgroup (launch_mfma in flash_fwd.hip) measured
-    faster than ``pick_fwd_splits``' workgroups and their combine. It is slower
-    only where few blocks have long rows (bf16, us, one launch / split: 12 heads
-    x 1024 x 8192 keys 51 / 44 at d = 64, 104 / 75 at 128; one causal head x
-    4096 54 / 37 at 128; 8 heads x 1024 x 4096 29 / 30 at 64; 16 heads x 1024 x
-    4096 55 / 60 at 128) and in even grids of 1 to 2 blocks a compute unit."""
+    """Key splits of a forward that names none: 1 where one launch of key
+    groups measured faster than ``pick_fwd_splits``' workgroups and their
+    combine (``_one_launch_keys``; in a window fewer of those hold live keys: 4
+    heads x 1024, 1024 of 6000 keys, d = 128, 22 / 40), and on causal grids of 1
+    to 1.5 blocks a compute unit, where the sweeps' lengths differ enough to leave units idle
+    (24 heads x 2048 causal, d = 128: 46 / 61 us; x 6000 keys, whose shortest
+    row sees 3953 of them, 161 / 139)."""
     if cus is None:
         cus = _cus()
     blocks = ninst * ((t + 127) // 128)
     lo, hi = (None, None) if band is None else (band.lo, band.hi)
     keys = s if lo is None or hi is None else min(s, hi - lo + 128)
-    if blocks <= cus and keys >= 256 and not (keys >= 8192 and 2 * blocks <= cus) and not (
-            d == 128 and keys >= 4096 and 4 * blocks <= cus):
+    if blocks <= cus and keys >= 256 and keys * keys < _one_launch_keys(256 * blocks / cus, d) * s:
         return 1
     if blocks > cus and (lo is None) != (hi is None) and 2 * blocks <= 3 * cus and keys >= 512:
-        return 1
+        shortest = hi + 1 if lo is None else s - max(t - 1 + lo, 0)  # live keys of the first (last) row
+        if 2 * shortest <= s:
+            return 1
     return pick_fwd_splits(ninst, t, s, cus)
 
 

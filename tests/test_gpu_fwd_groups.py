@@ -24,6 +24,48 @@ def test_key_splits_only_for_few_blocks_with_long_rows():
         assert _fwd_splits(n, t, s, d, band, cus=256) == pick_fwd_splits(n, t, s, cus=256)
 
 
+# (heads, t, keys, d, band): us of one launch and of the split, bf16, where they differ by a tenth
+MEASURED = {
+    (1, 1024, 1024, 64, None): (11.6, 16.4),
+    (1, 512, 3000, 64, None): (23.2, 16.9),
+    (1, 3000, 3000, 64, (None, 0)): (22.8, 20.5),
+    (1, 1024, 6000, 64, (None, 4976)): (39.2, 25.6),
+    (4, 256, 4096, 64, None): (28.0, 19.7),
+    (4, 1024, 6000, 64, (None, 4976)): (39.5, 34.3),
+    (8, 512, 6000, 64, None): (38.9, 33.4),
+    (8, 1024, 3000, 64, None): (23.3, 26.4),
+    (6, 3000, 3000, 64, None): (34.7, 30.7),
+    (12, 2048, 6000, 64, (None, 3952)): (63.0, 53.3),
+    (24, 1024, 6000, 64, None): (63.4, 54.2),
+    (12, 1024, 1024, 64, (None, 0)): (12.4, 19.7),
+    (8, 4096, 4096, 64, (None, 0)): (40.5, 45.4),
+    (1, 1500, 1500, 128, (None, 0)): (23.7, 18.6),
+    (1, 256, 2048, 128, None): (29.3, 17.5),
+    (2, 3000, 3000, 128, (None, 0)): (41.5, 29.9),
+    (4, 1024, 3000, 128, None): (42.0, 29.8),
+    (4, 512, 512, 128, (None, 0)): (12.5, 16.5),
+    (8, 2048, 6000, 128, None): (79.4, 65.7),
+    (12, 1024, 4096, 128, (None, 3072)): (55.0, 47.2),
+    (8, 2048, 2048, 128, None): (30.6, 39.5),
+    (12, 2048, 6000, 128, (None, 3952)): (98.3, 86.0),
+    (16, 2048, 2048, 128, None): (40.0, 54.7),
+    (24, 2048, 2048, 128, (None, 0)): (46.4, 60.8),
+    (24, 2048, 6000, 128, (None, 3952)): (161.0, 138.6),
+    (4, 1024, 6000, 128, (3953, 4976)): (22.3, 40.4),
+    (1, 4096, 4096, 128, (-1023, 0)): (20.6, 33.6),
+    (2, 512, 6000, 64, (4465, 5488)): (14.9, 27.7),
+    (4, 4177, 4177, 64, (None, 0)): (39.9, 34.6),
+}
+
+
+def test_the_faster_of_one_launch_and_a_split_is_taken():
+    from pdum_dsl_amd.kernels import Band, _fwd_splits
+
+    for (n, t, s, d, band), (one, split) in MEASURED.items():
+        got = _fwd_splits(n, t, s, d, None if band is None else Band(*band), cus=256)
+        assert (got == 1) == (one < split), (n, t, s, d, band, got)
+
+
 def _exact(q, k, v, band, fill, scale):
     """(o, sum p |v|, largest sum |q| |k|, lse) in float64."""
     q, k, v = (x.double().cpu() for x in (q, k, v))
