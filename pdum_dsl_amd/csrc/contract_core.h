@@ -567,8 +567,8 @@ __device__ __forceinline__ void contract_store(const ContractArgs& a, const pdh_
 // ds_read_b64_tr_b16; both arrive by direct loads of 1 KB. Returns with every
 // wave done with the operand tiles.
 // What bounds it: the loads and the products of a k tile overlap only in part.
-// 4096^3: 129 us, 86 without the loads, 94 without the products; 1024 x 768 x
-// 3072 (64 x 64 tiles, 48 k tiles): 16.5 us, 12.4, 13.3. Eight k tiles in flight,
+// 4096^3: 123 us, 81 without the loads, 92 without the products; 1024 x 768 x
+// 3072 (64 x 64 tiles, 48 k tiles): 15.0 us, 11.1, 11.3. Eight k tiles in flight,
 // two groups of four waves that split each k tile, and one workgroup of eight
 // waves with four 128-wide tiles in flight measured the same or slower.
 template <int DT, int WM, int LAY>
@@ -601,18 +601,11 @@ __device__ __forceinline__ void contract_mfma_loop(const ContractArgs& a, unsign
 
   // direct loads: 1 KB = 8 tile rows of 64 k values (lane i -> row i / 8, slot i % 8 holds chunk slot ^ swz(row)),
   // or RPK k rows of BM values (lane i -> row i / SLC, slot i % SLC)
-  const int lrow = lane >> 3, slot = lane & 7;
-  int ch[2];
-  uint32_t offa[2], offb[2];  // tile-row parity of the 8-row block decides the swizzle of row 8 j + lrow
+  const int lrow = lane >> 3, chunk = (lane & 7) ^ swz_gemm(8 * (w & 1) + lrow);  // this wave's 8-row blocks share the parity of w
   const int crow = lane / SLC, cswz = BM == 128 ? 4 * (crow & 3) : 4 * ((crow >> 1) & 1);
   const uint32_t cslot = static_cast<uint32_t>(((lane % SLC) ^ cswz) << 4);
-#pragma unroll
-  for (int par = 0; par < 2; ++par) {
-    ch[par] = slot ^ swz_gemm(8 * par + lrow);
-    const uint32_t sl = static_cast<uint32_t>(ch[par] << 4);
-    offa[par] = CA ? crow * rowa + cslot : lrow * rowa + sl;
-    offb[par] = CB ? crow * rowbb + cslot : lrow * rowbb + sl;
-  }
+  const uint32_t offa = CA ? crow * rowa + cslot : lrow * rowa + static_cast<uint32_t>(chunk << 4);
+  const uint32_t offb = CB ? crow * rowbb + cslot : lrow * rowbb + static_cast<uint32_t>(chunk << 4);
   // This wave's blocks of the next k tile to stage: scalar offsets into the
   // buffers and LDS, moved on by one add each (the loads of a k tile are
   // otherwise as much scalar work as the tile has products).
@@ -626,20 +619,16 @@ __device__ __forceinline__ void contract_mfma_loop(const ContractArgs& a, unsign
                 : static_cast<uint32_t>(n0 + 8 * blk) * rowbb;
   }
   const uint32_t stepa = CA ? kBK * rowa : kBK * 2u, stepb = CB ? kBK * rowbb : kBK * 2u;
-  int sk0 = 0, sbuf = 0;  // the next k tile's first k, its stage
-  auto stage = [&]() __attribute__((always_inline)) {  // stage s: a tile at 2 s, bt tile at 2 s + 1
-    const bool cut = sk0 + kBK > kin;  // the last, ragged k tile
-    const uint32_t lds = lds0 + sbuf * (2 * TILEB);
+  int sbuf;  // the next k tile's stage
+  auto stage = [&]() __attribute__((always_inline)) {
+    const uint32_t lds = lds0 + sbuf * (2 * TILEB);  // stage s: a tile at 2 s, bt tile at 2 s + 1
 #pragma unroll
     for (int i = 0; i < BLK; ++i) {
-      const int par = w & 1;
-      const bool out = cut && sk0 + 8 * ch[par] >= kin;
-      dma16_at(ar, lds + i * 4096, CA ? offa[0] : (out ? kOOB : offa[par]), soa[i]);
-      dma16_at(br, lds + TILEB + i * 4096, CB ? offb[0] : (out ? kOOB : offb[par]), sob[i]);
+      dma16_at(ar, lds + i * 4096, offa, soa[i]);
+      dma16_at(br, lds + TILEB + i * 4096, offb, sob[i]);
       soa[i] += stepa;
       sob[i] += stepb;
     }
-    sk0 += kBK;
     sbuf = sbuf + 1 == NS ? 0 : sbuf + 1;
   };
   // operand reads. k-contiguous: row (WM q + 32 t + r32) of a tile, chunk 2 ks + g
@@ -680,9 +669,23 @@ __device__ __forceinline__ void contract_mfma_loop(const ContractArgs& a, unsign
 #pragma unroll
     for (int j = 0; j < TI; ++j) acc[i][j] = f32x16{};
 
-  const int nkt = (kin + kBK - 1) / kBK;
+  // A ragged k tile (k no whole number of them) goes first, its row chunks past
+  // k moved out of the buffers. Handled at its place, the last, it was a choice at
+  // every load or a second copy of them in the loop: 1-8% for every k (512 x 2048 x
+  // 2048 11.6 us against 11.0, 1024 x 2048 x 1024 9.2 against 8.7, 4096^3 133
+  // against 127).
+  const int nkt = (kin + kBK - 1) / kBK, nfull = kin / kBK;
+  const bool ragged = nfull != nkt, past = ragged && nfull * kBK + 8 * chunk >= kin;
 #pragma unroll
-  for (int s = 0; s < NS - 1; ++s)
+  for (int i = 0; i < BLK; ++i) {
+    dma16_at(ar, lds0 + i * 4096, !CA && past ? kOOB : offa, soa[i] + (ragged ? nfull * stepa : 0u));
+    dma16_at(br, lds0 + TILEB + i * 4096, !CB && past ? kOOB : offb, sob[i] + (ragged ? nfull * stepb : 0u));
+    soa[i] += ragged ? 0u : stepa;
+    sob[i] += ragged ? 0u : stepb;
+  }
+  sbuf = 1;
+#pragma unroll
+  for (int s = 1; s < NS - 1; ++s)
     if (s < nkt) stage();
   int buf = 0;  // kt % NS
   for (int kt = 0; kt < nkt; ++kt, buf = buf + 1 == NS ? 0 : buf + 1) {
@@ -720,10 +723,10 @@ __device__ __forceinline__ void contract_mfma_loop(const ContractArgs& a, unsign
 // A workgroup's tile. XCD x (workgroups go round-robin over the eight) takes a
 // contiguous run of an order that walks groups of eight tile rows column by
 // column, so its L2 serves each bt panel to the whole group, and a k slice's
-// operands to its tiles (against row order, 1024 x 50257 x 768: 143 -> 107 us;
-// 458 x 320 x 6144 in six slices: 16.1 -> 12.7; 8192 x 3072 x 768: 54 -> 50; the
-// other shapes measured, 1024 x 768 x 768 to 4096^3, within 3%; groups of four
-// rows within 3% of eight).
+// operands to its tiles (against row order, 1024 x 50257 x 768: 143 -> 104 us;
+// 391 x 6466 x 1280: 20.7 -> 15.8; 458 x 320 x 6144 in six slices: 16.1 -> 12.7;
+// 8192 x 3072 x 768: 54 -> 50; the other shapes measured, 1024 x 768 x 768 to
+// 4096^3, within 3%; groups of four rows within 3% of eight).
 struct ContractTile {
   int b, tm, tn;
 };
