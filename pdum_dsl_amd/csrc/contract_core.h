@@ -738,7 +738,9 @@ __device__ __forceinline__ ContractTile contract_tile(const ContractArgs& a) {
   constexpr int GR = 8;
   const int grp = in_b / (GR * a.tiles_n), left = a.tiles_m - grp * GR, rows = left < GR ? left : GR;
   const int in = in_b - grp * GR * a.tiles_n;
-  return ContractTile{b, grp * GR + in % rows, in / rows};
+  // uniform, and kept scalar: the fp32 body otherwise ran up to 6% slower (below)
+  return ContractTile{__builtin_amdgcn_readfirstlane(b), __builtin_amdgcn_readfirstlane(grp * GR + in % rows),
+                      __builtin_amdgcn_readfirstlane(in / rows)};
 }
 
 template <int DT, int WM, typename Eval, int LAY = 0>
@@ -1003,10 +1005,11 @@ __device__ __forceinline__ void contract_split_body(const ContractArgs& a, const
   const int tid = threadIdx.x, lane = tid & 63, w = wave_id(), r32 = lane & 31, g = lane >> 5;
   const int wy = w >> 1, wx = w & 1;
   // contract_tile's order against row order (us, six products a term): 1024 x
-  // 50257 x 768 482 -> 454, 768 x 50257 x 1024 with both transposed 513 -> 475,
-  // 1024 x 768 x 50257 in 16 slices 502 -> 483, 12 x 1024 x 1024 x 64 19.7 ->
-  // 18.5; 4096^3 and 8192 x 3072 x 768 even, and grids under one workgroup per
-  // CU too (1024 x 768 x 768: 24.8 in row order, 24.7 so).
+  // 50257 x 768 469 -> 443, with both transposed 501 -> 465, 8192 x 3072 x 768 218 ->
+  // 214, 768 x 768 x 1024 in two slices 21.0 -> 20.2; on under 256 workgroups even
+  // (1024 x 768 x 768: 24.6, 24.3), or behind where bt alone is stored [k][n] (1024 x
+  // 768 x 3072 89.0 -> 91.5, 300 x 1000 x 513 19.0 -> 19.4; 94.8 and 20.2 before the
+  // tile's coordinates were kept scalar).
   const ContractTile tl = contract_tile(a);
   const int b = tl.b, m0 = tl.tm * BM, n0 = tl.tn * BM;
   const float* abase = static_cast<const float*>(a.a) + contract_off_a(a, b);
