@@ -24,9 +24,10 @@
 // enough reuse, and it leaves the small blocks that balance a causal sweep
 // over 256 CUs. Against the VALU kernels this replaced (one wave per row; one
 // row per lane in the forward): 24 causal heads x 1000, D = 64, backward 7070
-// -> 163 us and forward 182 -> 58 us; 32 heads x 2048, D = 64, all keys live:
-// forward 119 TFLOP/s, backward 109 (seven products, the dQ role recomputes
-// two) of the 157 the fp32 matrix cores peak at; one head x 256: 29 -> 7.3 us.
+// -> 157 us and forward 182 -> 56 us (matrix pipe 48% and 36% busy: the causal
+// tail); 32 heads x 2048, D = 64, all keys live: forward 115 TFLOP/s, backward 117
+// (seven products, the dQ role recomputes two) of the 157 the fp32 matrix cores
+// peak at, 72% and 75% busy; one head x 256: 29 -> 7.2 us.
 // The distance to 64 bits is smaller than the VALU kernels' (o 1.8e-7, dK 3.9e-7 of
 // the norm at 24 x 1000, against 2.6e-7 and 8.1e-7).
 #include "attn_f32.h"

@@ -28,7 +28,8 @@ int compute_units() {
 // short; otherwise the cheapest under what a slice costs: a 64-wide k tile
 // takes kTile us, the finish kFin us plus its planes' traffic. 458 x 320 x
 // 6144 (40 tiles): 28.2 -> 12.7 us; 64 x 512 x 4096 (8): 19.7 -> 11.1; 24 x 6144
-// x 4096 (96): 19.9 -> 15.5.
+// x 4096 (96): 19.9 -> 15.5. Over half a tile per compute unit two slices pass one
+// workgroup a unit and are not taken; two a unit have not been measured.
 int pick_split(int64_t batch, int64_t m, int64_t n, int64_t k) {
   constexpr double kTile = 0.27, kFin = 3.5, kBytesPerUs = 4e6;
   const int64_t tiles = batch * ((m + 63) / 64) * ((n + 63) / 64), kt = (k + kBK - 1) / kBK;

@@ -986,7 +986,9 @@ int launch_as(const FwdArgs& a, int64_t ninst, hipStream_t st) {
 //   38 x 1024 c x 128        39.9    47.1   32.4 (2, 2)
 //   32 x 4096 c x 64        126.2      -    93.7 (2, 2)
 //   64 x 2048 c x 64         72.2      -    63.5 (2, 2);  x 128: 106.6, 107.2 kept
-// and past the lines: 64 x 1024 c x 64: 26.1 (4, 1), 28.0 (2, 2); 50 x 1024 x
+// One line for all of D = 64 up to half a block per unit and one for the rest:
+// (2, 4) would be 7% better at 16 x 2048 c x 64 and 24% worse at 24 x 1024 x 2048.
+// And past the lines: 64 x 1024 c x 64: 26.1 (4, 1), 28.0 (2, 2); 50 x 1024 x
 // 1024 x 64: 24.8, 29.6; 128 x 2048 c x 64: 100.2, 109.8; 53 keys: 5.4, 6.7.
 template <typename T, int D>
 int launch_mfma(const FwdArgs& a, int64_t ninst, hipStream_t st) {
